@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/isph_capi.h"
+#include "isph_gridsync.h"
 #include "isph_kernels.h"
 
 using namespace isph;
@@ -459,13 +460,26 @@ KrylovArgs<TV, TX, TI> krylov_args(isph_ctx* c, const TI* nbr, const TV* val, TX
     return a;
 }
 
+// iterations per launch of a resident solve: a launch ends within tens of
+// milliseconds, and the next one carries on from the state it left
+constexpr int RESIDENT_ITERS = 4096;
+
 // BiCGSTAB iterations in batches until the device sets sc->done; the host
-// polls after each batch.  `first` selects p = r for the first iteration
-// after a (re)start.  prof slots k0, k0+1: the two SpMV kernels.
+// polls after each batch.  Systems that fit on the chip iterate inside one
+// launch instead (not while the SpMV launches are being timed).  `first`
+// selects p = r for the first iteration after a (re)start.  prof slots k0,
+// k0+1: the two SpMV kernels.
 template <class TV, class TX, class TI>
 int iterate(isph_ctx* c, const KrylovArgs<TV, TX, TI>& a, const SolveCtl& ctl, bool& first,
             int k0) {
     const int grid = nblk8(c->n);
+    if constexpr (std::is_same<TI, short>::value) {
+        for (bool resident = !c->prof.on; resident;) {
+            int rc = resident_iterate<TV, TX>(c, a, ctl, first, RESIDENT_ITERS, resident);
+            if (rc) return rc;
+            if (resident && c->sc_host->done) return ISPH_OK;
+        }
+    }
     for (;;) {
         const int before = c->sc_host->total;
         int batch = 8;
@@ -756,6 +770,12 @@ int isph_create(const isph_params* prm, int32_t cap, int32_t cap_soil, isph_ctx*
         delete c;
         return ISPH_E_HIP;
     }
+    int coop = 0;
+    if (hipGetDevice(&c->device) == hipSuccess &&
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device) == hipSuccess &&
+        hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device) ==
+            hipSuccess)
+        c->cooperative = coop != 0;
     // the device address of this GPU's isph_probe_noalloc scratch array
     if ((rc = probe_scratch_attach(c))) {
         (void)hipStreamDestroy(c->stream);
@@ -796,9 +816,10 @@ int isph_create(const isph_params* prm, int32_t cap, int32_t cap_soil, isph_ctx*
     rc |= dalloc(c, &c->rv32, N);
     rc |= dalloc(c, &c->part, 4 * (size_t)nblk8(cap));
     rc |= dalloc(c, &c->counters, 16);
+    rc |= dalloc(c, &c->gs_words, (size_t)GS_WORDS);
     rc |= dalloc(c, &c->sc, 1);
     rc |= dalloc(c, &c->ss, 1);
-    rc |= dalloc(c, &c->err, 1);
+    rc |= dalloc(c, &c->err, 2);
     rc |= dalloc(c, &c->spos, (size_t)std::max(cap_soil, 1));
     rc |= dalloc(c, &c->smass, (size_t)std::max(cap_soil, 1));
     rc |= dalloc(c, &c->srho, (size_t)std::max(cap_soil, 1));
@@ -835,6 +856,7 @@ int isph_destroy(isph_ctx* c) {
                  c->bincnt, c->scanbuf, c->nbr16,
                  c->rq64, c->rv64, c->rq32, c->rv32, c->rsum,
                  c->nbr, c->cnt, c->val64, c->val32, c->dpos, c->rhs, c->part, c->counters,
+                 c->gs_words,
                  c->sc, c->ss, c->err, c->spos, c->smass, c->srho, c->sstart,
                  c->pos_nb, c->cdiff, c->salt_coef, c->fsol};
     for (auto q : p)

@@ -1,0 +1,129 @@
+// isph_gridsync.h -- grid-wide sums for kernels whose blocks all stay resident
+// (cooperative launches).  Worker blocks publish their part of a sum; one more
+// block, the leader, reads all parts, finishes the reduction and broadcasts
+// what the workers need of it.  The exchange is reduction and barrier in one.
+//
+// Every published 64-bit word carries 32 bits of data under a 32-bit epoch
+// number, so it is valid by itself and no flag has to follow the data.  Words
+// are written and read with agent-scope atomics, which go past the XCDs'
+// private L2 caches.  Two buffers alternate by epoch: a worker publishes epoch
+// e + 2 only after the broadcast of e + 1, for which the leader needed every
+// worker's part of e + 1, and a worker publishes that after it has read the
+// broadcast of e; likewise for the leader's words.  The words are zeroed
+// before each launch and epochs count from 1.
+//
+// Vector entries that other blocks read after an exchange are stored with
+// agent-scope atomics (write-through, so nothing has to be written back) and
+// are complete (vmcnt 0) before the block publishes; the readers load them
+// with agent-scope atomics after the exchange.  No cache is written back or
+// invalidated: at 256 blocks an exchange costs 2.0 us this way, 14 us with a
+// release and an acquire fence of agent scope, and 3.4 us if every block reads
+// every part itself.
+//
+// Every wait is bounded (GS_SPIN polls, about a second): a block that gives up
+// raises ERR_SYNC and ends, the others run into their own bounds, and the grid
+// drains.
+#pragma once
+#include "isph_kernels.h"
+
+namespace isph {
+
+constexpr int GS_MAXB = 256;      // blocks of a resident grid, one per CU, the leader included
+constexpr int GS_LINES = 32;      // copies of the broadcast, one per 128-byte line
+constexpr int GS_LINE = 16;       // words of a line
+constexpr int GS_SPIN = 1 << 20;  // polls before a block gives up
+// words of both buffers: 4 per worker, then the broadcast lines
+constexpr int GS_WORDS = 2 * (4 * GS_MAXB + GS_LINES * GS_LINE);
+
+typedef unsigned long long gs_word;
+
+struct GridSync {
+    gs_word* words;
+    uint32_t* err;
+};
+
+__device__ __forceinline__ gs_word* gs_part(const GridSync& g, uint32_t e, int block) {
+    return g.words + (size_t)(e & 1) * 4 * GS_MAXB + block;
+}
+__device__ __forceinline__ gs_word* gs_line(const GridSync& g, uint32_t e, int line) {
+    return g.words + 2 * 4 * GS_MAXB + ((size_t)(e & 1) * GS_LINES + line) * GS_LINE;
+}
+
+template <class T>
+__device__ __forceinline__ void gs_store(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ T gs_load(const T* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ gs_word gs_hi(uint32_t e, double v) {
+    return ((gs_word)e << 32) | ((gs_word)__double_as_longlong(v) >> 32);
+}
+__device__ __forceinline__ gs_word gs_lo(uint32_t e, double v) {
+    return ((gs_word)e << 32) | ((gs_word)__double_as_longlong(v) & 0xffffffffull);
+}
+__device__ __forceinline__ double gs_value(gs_word hi, gs_word lo) {
+    return __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
+}
+
+// worker: one thread publishes the block's parts of epoch e
+__device__ __forceinline__ void gs_publish(const GridSync& g, uint32_t e, int block, bool two,
+                                           double v0, double v1) {
+    gs_word* w = gs_part(g, e, block);
+    gs_store(w, gs_hi(e, v0));
+    gs_store(w + GS_MAXB, gs_lo(e, v0));
+    if (two) {
+        gs_store(w + 2 * GS_MAXB, gs_hi(e, v1));
+        gs_store(w + 3 * GS_MAXB, gs_lo(e, v1));
+    }
+}
+
+// leader: a thread reads worker b's parts of epoch e; false if they did not come
+__device__ __forceinline__ bool gs_collect(const GridSync& g, uint32_t e, int b, bool two,
+                                           double& v0, double& v1) {
+    const gs_word* w = gs_part(g, e, b);
+    for (int spin = 0; spin < GS_SPIN; ++spin) {
+        const gs_word a = gs_load(w), c = gs_load(w + GS_MAXB);
+        const gs_word d = two ? gs_load(w + 2 * GS_MAXB) : a;
+        const gs_word f = two ? gs_load(w + 3 * GS_MAXB) : a;
+        if ((uint32_t)(a >> 32) == e && (uint32_t)(c >> 32) == e && (uint32_t)(d >> 32) == e &&
+            (uint32_t)(f >> 32) == e) {
+            v0 = gs_value(a, c);
+            v1 = two ? gs_value(d, f) : 0.0;
+            return true;
+        }
+    }
+    return false;
+}
+
+// leader: threads 0 .. GS_LINES - 1 broadcast a value and a flag
+__device__ __forceinline__ void gs_broadcast(const GridSync& g, uint32_t e, double v, int flag) {
+    if (threadIdx.x < GS_LINES) {
+        gs_word* w = gs_line(g, e, threadIdx.x);
+        gs_store(w, gs_hi(e, v));
+        gs_store(w + 1, gs_lo(e, v));
+        gs_store(w + 2, ((gs_word)e << 32) | (uint32_t)flag);
+    }
+}
+
+// worker: every wave reads the broadcast of epoch e for itself
+__device__ __forceinline__ bool gs_receive(const GridSync& g, uint32_t e, int block, double& v,
+                                           int& flag) {
+    const int lane = threadIdx.x & 63;
+    const gs_word* w = gs_line(g, e, block & (GS_LINES - 1)) + min(lane, 2);
+    for (int spin = 0; spin < GS_SPIN; ++spin) {
+        const gs_word x = gs_load(w);
+        if (__all((uint32_t)(x >> 32) == e)) {
+            const gs_word hi = __shfl(x, 0, 64), lo = __shfl(x, 1, 64), f = __shfl(x, 2, 64);
+            v = gs_value(hi, lo);
+            flag = (int)(uint32_t)f;
+            // keeps the compiler from moving later loads up; no cache action
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            return true;
+        }
+    }
+    return false;
+}
+
+}  // namespace isph

@@ -86,7 +86,10 @@ struct isph_ctx {
     isph::SolverScalars* sc_host = nullptr;  // pinned
     isph::SimScalars* ss = nullptr;
     isph::SimScalars* ss_host = nullptr;  // pinned
-    uint32_t* err = nullptr;
+    uint32_t* err = nullptr;       // error bits; [1]: a resident solve refused the system
+    int device = 0, cus = 0;       // GPU of the context, its compute units
+    bool cooperative = false;      // it takes cooperative launches
+    unsigned long long* gs_words = nullptr;  // exchange words of the resident solves
     double2* pos_nb = nullptr;     // positions at the last neighbour search
     double* cdiff = nullptr;       // salinity rate of the last scalart
     double4* salt_coef = nullptr;  // per particle (Dx, Dy, Dm + nut/ts, nut)
@@ -192,6 +195,16 @@ int run_step(isph_ctx* c);
 // (unit diagonal at dpos) and right-hand side; x holds the initial guess
 // on entry and the solution on return.
 int solve_fp64_on(isph_ctx* c, const double* val, const double* rhs, double* x);
+
+// Up to maxiter BiCGSTAB iterations in one cooperative launch
+// (isph_resident.hip); on return sc_host holds the state and `first` is
+// cleared.  `ran` is false, and nothing has changed, when the system is too
+// large, its rows reach too far, or the GPU cannot hold the grid.  (Offsets
+// that do not fit 16 bits reach too far.)
+constexpr size_t RESIDENT_LDS = 154 * 1024;  // of a CU's 160 KB, beside the static shared memory
+template <class TV, class TX>
+int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
+                     bool& first, int maxiter, bool& ran);
 
 // solver pieces shared with the multigrid solve (isph_mg.hip)
 __global__ void k_fill(int n, double* x, double v);

@@ -25,6 +25,7 @@ constexpr uint32_t ERR_SINGULAR = 8u;
 constexpr uint32_t ERR_NOCONV = 16u;
 constexpr uint32_t ERR_INDEX16 = 32u;  // a column offset does not fit 16 bits
 constexpr uint32_t ERR_SUBSTEPS = 64u; // salinity transport needs > MAX_SUBSTEPS substeps
+constexpr uint32_t ERR_SYNC = 128u;    // a block of a resident grid waited in vain
 
 // cap on the transport substeps of one step (integrator.f90:966-970 has none;
 // its ceiling() would overflow a default integer long before this)
@@ -126,11 +127,44 @@ constexpr double BRK_COS = 1e-15;
 // fixed-tree reductions: wave64 butterfly (xor 1,2,..,32), then the four
 // waves of a 256-thread block as (w0+w1)+(w2+w3)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int s = 1; s < 64; s <<= 1) v = v + __shfl_xor(v, s, 64);
+template <int CTRL>
+__device__ __forceinline__ double lane_move(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// The butterfly v + v[lane ^ s], s = 1, 2, .., N / 2, in aligned groups of N
+// lanes, without LDS: lanes that already hold the same value may stand in for
+// each other, so a quad permutation makes s = 1 and 2, mirrors of 8 and 16
+// lanes make 4 and 8, and the row swaps make 16 and 32 (each lane adds the two
+// rows' values; addition commutes).  Same bits as the shuffles, which take an
+// LDS round trip a step.
+template <int N>
+__device__ __forceinline__ double lanes_sum(double v) {
+    v = v + lane_move<0xB1>(v);                // quad_perm 1,0,3,2
+    v = v + lane_move<0x4E>(v);                // quad_perm 2,3,0,1
+    if (N >= 8) v = v + lane_move<0x141>(v);   // row_half_mirror
+    if (N >= 16) v = v + lane_move<0x140>(v);  // row_mirror
+    if (N >= 32) {
+        const long long b = __double_as_longlong(v);
+        const auto lo = __builtin_amdgcn_permlane16_swap((int)b, (int)b, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((int)(b >> 32), (int)(b >> 32), false, false);
+        v = __longlong_as_double(((long long)hi[0] << 32) | (unsigned int)lo[0]) +
+            __longlong_as_double(((long long)hi[1] << 32) | (unsigned int)lo[1]);
+    }
+    if (N >= 64) {
+        const long long b = __double_as_longlong(v);
+        const auto lo = __builtin_amdgcn_permlane32_swap((int)b, (int)b, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((int)(b >> 32), (int)(b >> 32), false, false);
+        v = __longlong_as_double(((long long)hi[0] << 32) | (unsigned int)lo[0]) +
+            __longlong_as_double(((long long)hi[1] << 32) | (unsigned int)lo[1]);
+    }
     return v;
 }
+
+__device__ __forceinline__ double wave_sum(double v) { return lanes_sum<64>(v); }
 
 // block sum in the fixed tree; the result is valid in every thread
 __device__ __forceinline__ double block_sum(double v) {

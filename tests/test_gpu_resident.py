@@ -1,0 +1,83 @@
+"""BiCGSTAB in one cooperative launch (csrc/isph_resident.hip) against the
+launched kernels: timing the SpMV launches (profile_enable) selects the
+latter.  Same arithmetic in the same order, so every bit agrees."""
+import numpy as np
+import pytest
+
+from beach_slope_confined_amd import capi, configs
+from beach_slope_confined_amd.params import PREC_FP64, PREC_IR, PREC_MIXED_V64
+
+pytestmark = pytest.mark.gpu
+
+
+def _step(cfg, launched):
+    sim = configs.make_sim(cfg, capi.IsphSim)
+    if launched:
+        sim.profile_enable(1)
+    sim.step(1)
+    s, q = sim.scalars(), sim.get_particles()
+    timed = sim.kernel_time(0)[0] + sim.kernel_time(2)[0]
+    sim.close()
+    return s, q, timed
+
+
+def _same(cfg, **changes):
+    cfg = dict(cfg, params=cfg["params"].copy(**changes))
+    s0, q0, timed = _step(cfg, True)
+    s1, q1, _ = _step(cfg, False)
+    assert timed > 0  # the first run's SpMVs were launches
+    assert (s0["iters"], s0["outer"], s0["relres"]) == (s1["iters"], s1["outer"], s1["relres"])
+    for k in q0:
+        assert np.array_equal(q0[k], q1[k]), k
+
+
+# (nside + 6)(nside + 3) rows: less than a block, blocks of 256, 512 and 1024
+# rows on both sides of where one gives way to the next, and just too large
+@pytest.mark.parametrize("nside", [8, 64, 251, 252, 356, 357, 506, 507])
+def test_fp64_sizes(require_gpu, nside):
+    _same(configs.tank_1m(nside), precision=PREC_FP64)
+
+
+@pytest.mark.parametrize("nside", [40, 252, 357])
+def test_mixed_with_updates(require_gpu, nside):
+    _same(configs.tank_1m(nside), precision=PREC_MIXED_V64)
+
+
+def test_fp32_vectors(require_gpu):
+    _same(configs.tank_1m(64), precision=PREC_IR)
+
+
+def test_more_iterations_than_one_launch(require_gpu):
+    _same(configs.dam_break(0.001), precision=PREC_FP64)
+
+
+@pytest.mark.parametrize("cells", [2.0, 16.0])
+def test_rows_that_reach_far(require_gpu, cells):
+    """Particles in random order in large cells: a block's rows refer to
+    rows all over their cells, past what a block can carry."""
+    cfg = configs.dam_break(0.005)
+    rng = np.random.default_rng(3)
+    o = rng.permutation(len(cfg["parts"]["x"]))
+    cfg["parts"] = {k: np.ascontiguousarray(v[o]) for k, v in cfg["parts"].items()}
+    _same(cfg, cell_size=cells * cfg["params"].h)
+
+
+def test_two_threads(require_gpu):
+    """Two contexts solving at the same time: their grids must not share the
+    chip half and half."""
+    import threading
+    cfg = configs.tank_1m(200)
+    _, ref, _ = _step(cfg, False)
+    out = [None, None]
+
+    def work(k):
+        for _ in range(3):
+            out[k] = _step(cfg, False)[1]
+    th = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for x in th:
+        x.start()
+    for x in th:
+        x.join()
+    for q in out:
+        for k in ref:
+            assert np.array_equal(ref[k], q[k]), k
