@@ -816,7 +816,7 @@ int isph_create(const isph_params* prm, int32_t cap, int32_t cap_soil, isph_ctx*
     rc |= dalloc(c, &c->rv32, N);
     rc |= dalloc(c, &c->part, 4 * (size_t)nblk8(cap));
     rc |= dalloc(c, &c->counters, 16);
-    rc |= dalloc(c, &c->gs_words, (size_t)GS_WORDS);
+    rc |= dalloc(c, &c->gs_words, (size_t)gs_words(GS_PARTS));
     rc |= dalloc(c, &c->sc, 1);
     rc |= dalloc(c, &c->ss, 1);
     rc |= dalloc(c, &c->err, 2);

@@ -29,24 +29,30 @@
 namespace isph {
 
 constexpr int GS_MAXB = 256;      // blocks of a resident grid, one per CU, the leader included
+constexpr int GS_PARTS = 5120 + 256;  // published parts of a sum, and room for partial sums
 constexpr int GS_LINES = 32;      // copies of the broadcast, one per 128-byte line
 constexpr int GS_LINE = 16;       // words of a line
 constexpr int GS_SPIN = 1 << 20;  // polls before a block gives up
-// words of both buffers: 4 per worker, then the broadcast lines
-constexpr int GS_WORDS = 2 * (4 * GS_MAXB + GS_LINES * GS_LINE);
 
 typedef unsigned long long gs_word;
 
+// words of both buffers: the broadcast lines, then 4 per part
+constexpr int gs_words(int parts) { return 2 * (GS_LINES * GS_LINE + 4 * parts); }
+
 struct GridSync {
     gs_word* words;
-    uint32_t* err;
+    uint32_t* err;    // error bits
+    uint32_t* state;  // GS_REFUSED, GS_WRITTEN; cleared with the words
+    int parts;        // a multiple of 256
 };
+constexpr uint32_t GS_REFUSED = 1u;  // some block cannot hold its rows: nothing was done
+constexpr uint32_t GS_WRITTEN = 2u;  // a block has written its part of the result
 
-__device__ __forceinline__ gs_word* gs_part(const GridSync& g, uint32_t e, int block) {
-    return g.words + (size_t)(e & 1) * 4 * GS_MAXB + block;
+__device__ __forceinline__ gs_word* gs_part(const GridSync& g, uint32_t e, int part) {
+    return g.words + 2 * GS_LINES * GS_LINE + (size_t)(e & 1) * 4 * g.parts + part;
 }
 __device__ __forceinline__ gs_word* gs_line(const GridSync& g, uint32_t e, int line) {
-    return g.words + 2 * 4 * GS_MAXB + ((size_t)(e & 1) * GS_LINES + line) * GS_LINE;
+    return g.words + ((size_t)(e & 1) * GS_LINES + line) * GS_LINE;
 }
 
 template <class T>
@@ -67,30 +73,44 @@ __device__ __forceinline__ double gs_value(gs_word hi, gs_word lo) {
     return __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
 }
 
-// worker: one thread publishes the block's parts of epoch e
-__device__ __forceinline__ void gs_publish(const GridSync& g, uint32_t e, int block, bool two,
+// worker: a thread publishes one part of epoch e
+__device__ __forceinline__ void gs_publish(const GridSync& g, uint32_t e, int part, bool two,
                                            double v0, double v1) {
-    gs_word* w = gs_part(g, e, block);
+    gs_word* w = gs_part(g, e, part);
     gs_store(w, gs_hi(e, v0));
-    gs_store(w + GS_MAXB, gs_lo(e, v0));
+    gs_store(w + g.parts, gs_lo(e, v0));
     if (two) {
-        gs_store(w + 2 * GS_MAXB, gs_hi(e, v1));
-        gs_store(w + 3 * GS_MAXB, gs_lo(e, v1));
+        gs_store(w + 2 * g.parts, gs_hi(e, v1));
+        gs_store(w + 3 * g.parts, gs_lo(e, v1));
     }
 }
 
-// leader: a thread reads worker b's parts of epoch e; false if they did not come
-__device__ __forceinline__ bool gs_collect(const GridSync& g, uint32_t e, int b, bool two,
-                                           double& v0, double& v1) {
-    const gs_word* w = gs_part(g, e, b);
+// leader: a thread reads the N parts first, first + stride, .. of epoch e that
+// lie below `count` (the others are 0); false if one did not come
+template <int N>
+__device__ __forceinline__ bool gs_collect(const GridSync& g, uint32_t e, int first, int stride,
+                                           int count, bool two, double* v0, double* v1) {
     for (int spin = 0; spin < GS_SPIN; ++spin) {
-        const gs_word a = gs_load(w), c = gs_load(w + GS_MAXB);
-        const gs_word d = two ? gs_load(w + 2 * GS_MAXB) : a;
-        const gs_word f = two ? gs_load(w + 3 * GS_MAXB) : a;
-        if ((uint32_t)(a >> 32) == e && (uint32_t)(c >> 32) == e && (uint32_t)(d >> 32) == e &&
-            (uint32_t)(f >> 32) == e) {
-            v0 = gs_value(a, c);
-            v1 = two ? gs_value(d, f) : 0.0;
+        gs_word x[N][4];
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            const bool in = first + m * stride < count;
+            const gs_word* w = gs_part(g, e, in ? first + m * stride : first);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                x[m][q] = in && (q < 2 || two) ? gs_load(w + q * g.parts) : (gs_word)e << 32;
+        }
+        bool ok = true;
+#pragma unroll
+        for (int m = 0; m < N; ++m)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ok = ok && (uint32_t)(x[m][q] >> 32) == e;
+        if (ok) {
+#pragma unroll
+            for (int m = 0; m < N; ++m) {
+                v0[m] = gs_value(x[m][0], x[m][1]);
+                v1[m] = gs_value(x[m][2], x[m][3]);
+            }
             return true;
         }
     }

@@ -1,0 +1,49 @@
+// isph_gridsync.hip -- launching grids whose blocks wait for each other.
+#include "isph_gridsync.h"
+#include "isph_host.h"
+
+namespace isph {
+
+__global__ void k_gs_clear(int n, gs_word* w, uint32_t* state) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i < n) w[i] = 0ull;
+    if (i == 0) *state = 0;
+}
+
+namespace host {
+
+int grid_launch(isph_ctx* c, const void* kern, int blocks, int threads, void** args, size_t lds,
+                int parts, bool& ran) {
+    ran = false;
+    if (lds > 64 * 1024)
+        HIPCHK(c, hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int n = gs_words(parts);
+    k_gs_clear<<<nblk(n), BLOCK, 0, c->stream>>>(n, c->gs_words, c->err + 1);
+    const hipError_t e = hipLaunchCooperativeKernel(kern, dim3(blocks), dim3(threads), args,
+                                                    (unsigned)lds, c->stream);
+    if (e != hipSuccess) {
+        // One process at a time holds a GPU's cooperative queue; a second one
+        // is refused, and its contexts keep to the launched kernels.
+        (void)hipGetLastError();
+        c->cooperative = false;
+        return ISPH_OK;
+    }
+    uint32_t word[2] = {0, 0};
+    HIPCHK(c, hipMemcpyAsync(word, c->err, sizeof(word), hipMemcpyDeviceToHost, c->stream));
+    if (int rc = read_sc(c)) return rc;
+    if (word[0] & ERR_SYNC) {
+        // Blocks waited in vain: something else holds their CUs.  Unless one
+        // has written its part back, the launched kernels carry on from the
+        // state the launch began with, from now on.
+        c->cooperative = false;
+        HIPCHK(c, hipMemsetAsync(c->err, 0, sizeof(uint32_t), c->stream));
+        if (word[1] & GS_WRITTEN) return fail(c, ISPH_E_HIP, "a resident solve lost a block");
+        return ISPH_OK;
+    }
+    if (word[1] & GS_REFUSED) return ISPH_OK;
+    ran = true;
+    return ISPH_OK;
+}
+
+}  // namespace host
+}  // namespace isph

@@ -86,7 +86,7 @@ struct isph_ctx {
     isph::SolverScalars* sc_host = nullptr;  // pinned
     isph::SimScalars* ss = nullptr;
     isph::SimScalars* ss_host = nullptr;  // pinned
-    uint32_t* err = nullptr;       // error bits; [1]: a resident solve refused the system
+    uint32_t* err = nullptr;       // error bits; [1]: a resident solve's GS_* state
     int device = 0, cus = 0;       // GPU of the context, its compute units
     bool cooperative = false;      // it takes cooperative launches
     unsigned long long* gs_words = nullptr;  // exchange words of the resident solves
@@ -201,10 +201,19 @@ int solve_fp64_on(isph_ctx* c, const double* val, const double* rhs, double* x);
 // cleared.  `ran` is false, and nothing has changed, when the system is too
 // large, its rows reach too far, or the GPU cannot hold the grid.  (Offsets
 // that do not fit 16 bits reach too far.)
-constexpr size_t RESIDENT_LDS = 154 * 1024;  // of a CU's 160 KB, beside the static shared memory
+constexpr size_t RESIDENT_LDS = 152 * 1024;  // of a CU's 160 KB, beside the static shared memory
 template <class TV, class TX>
 int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
                      bool& first, int maxiter, bool& ran);
+
+// the same for larger systems, the matrix read from memory (isph_streamed.hip)
+template <class TV, class TX>
+int streamed_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
+                     bool& first, int maxiter, bool& ran);
+// Launches a resident grid that leaves the solver state in c->sc and waits for
+// it (sc_host); `ran` as in resident_iterate.
+int grid_launch(isph_ctx* c, const void* kern, int blocks, int threads, void** args, size_t lds,
+                int parts, bool& ran);
 
 // solver pieces shared with the multigrid solve (isph_mg.hip)
 __global__ void k_fill(int n, double* x, double v);

@@ -168,14 +168,14 @@ __device__ __forceinline__ void resident_leader(const GridSync& gs, double (*red
     uint32_t e = 1;
     {
         double a = 0.0, b = 0.0;
-        if (t < nw && !gs_collect(gs, e, t, false, a, b)) *lost = 1;
+        if (t < nw && !gs_collect<1>(gs, e, t, 0, nw, false, &a, &b)) *lost = 1;
         if (a != 0.0) *lost = 2;
     }
     __syncthreads();
     const int refused = *lost;
     gs_broadcast(gs, e, 0.0, refused);
     if (refused) {
-        if (t == 0) refused == 1 ? atomicOr(gs.err, ERR_SYNC) : atomicOr(gs.err + 1, 1u);
+        if (t == 0) refused == 1 ? atomicOr(gs.err, ERR_SYNC) : atomicOr(gs.state, GS_REFUSED);
         return;
     }
     for (int it = 0; it < maxiter; ++it) {
@@ -184,7 +184,7 @@ __device__ __forceinline__ void resident_leader(const GridSync& gs, double (*red
             ++e;
             const bool two = kind != FIN_ALPHA;
             double a = 0.0, b = 0.0;
-            if (t < nw && !gs_collect(gs, e, t, two, a, b)) *lost = 1;
+            if (t < nw && !gs_collect<1>(gs, e, t, 0, nw, two, &a, &b)) *lost = 1;
             a = lanes_sum<PER>(a);
             b = lanes_sum<PER>(b);
             if (t % PER == 0) {
@@ -401,6 +401,7 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         atomicOr(gs.err, ERR_SYNC);
         return;
     }
+    if (t == 0) atomicOr(gs.state, GS_WRITTEN);
     if (own) {
         a.xs[i] = x;
         P2 u;
@@ -409,9 +410,6 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         a.rq[i] = u;
     }
 }
-
-__global__ void k_gs_clear(gs_word* w) { w[blockIdx.x * BLOCK + threadIdx.x] = 0ull; }
-static_assert(GS_WORDS % BLOCK == 0, "whole blocks clear the words");
 
 namespace host {
 
@@ -427,46 +425,14 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
     constexpr size_t per = (sizeof(TV) + sizeof(unsigned short)) * R;
     const int kl = (int)std::min<size_t>((size_t)c->prm.max_nbr, (RESIDENT_LDS - win) / per);
     const size_t lds = win + per * kl;
-    if (lds > 64 * 1024)
-        HIPCHK(c, hipFuncSetAttribute((const void*)kern,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     KrylovArgs<TV, TX, short> a = ka;
-    GridSync gs{c->gs_words, c->err};
+    GridSync gs{c->gs_words, c->err, c->err + 1, GS_MAXB};
     SolverScalars* sc = c->sc;
     SolveCtl t = ctl;
     int f = first, m = maxiter, l = kl;
-    k_gs_clear<<<GS_WORDS / BLOCK, BLOCK, 0, c->stream>>>(c->gs_words);
     void* args[] = {&a, &gs, &sc, &t, &f, &m, &l};
-    const hipError_t e = hipLaunchCooperativeKernel((const void*)kern, dim3(blocks), dim3(R), args,
-                                                    (unsigned)lds, c->stream);
-    if (e != hipSuccess) {
-        // One process at a time holds a GPU's cooperative queue; a second one
-        // is refused, and its contexts keep to the launched kernels.
-        (void)hipGetLastError();
-        c->cooperative = false;
-        return ISPH_OK;
-    }
-    const int before = c->sc_host->total;
-    uint32_t word[2] = {0, 0};
-    HIPCHK(c, hipMemcpyAsync(word, c->err, sizeof(word), hipMemcpyDeviceToHost, c->stream));
-    if (int rc = read_sc(c)) return rc;
-    if (word[1]) {  // a block's window did not fit
-        HIPCHK(c, hipMemsetAsync(c->err + 1, 0, sizeof(uint32_t), c->stream));
-        return ISPH_OK;
-    }
-    if (word[0] & ERR_SYNC) {
-        // Blocks waited in vain: something else holds their CUs.  The leader
-        // gave up before its last broadcast (it stores the scalars after it),
-        // so no block has written anything back and the launched kernels
-        // carry on from the same state, from now on.
-        c->cooperative = false;
-        HIPCHK(c, hipMemsetAsync(c->err, 0, sizeof(uint32_t), c->stream));
-        if (c->sc_host->total != before)
-            return fail(c, ISPH_E_HIP, "a resident solve lost a block");
-        return ISPH_OK;
-    }
-    first = false;
-    ran = true;
+    if (int rc = grid_launch(c, (const void*)kern, blocks, R, args, lds, GS_MAXB, ran)) return rc;
+    if (ran) first = false;
     return ISPH_OK;
 }
 
@@ -482,7 +448,7 @@ int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const Solv
     if (nb <= most) return launch<TV, TX, 1>(c, a, ctl, first, maxiter, ran);
     if (nb <= 2 * most) return launch<TV, TX, 2>(c, a, ctl, first, maxiter, ran);
     if (nb <= 4 * most) return launch<TV, TX, 4>(c, a, ctl, first, maxiter, ran);
-    return ISPH_OK;
+    return streamed_iterate<TV, TX>(c, a, ctl, first, maxiter, ran);
 }
 
 #define ISPH_RESIDENT(TV, TX)                                                                  \

@@ -31,9 +31,12 @@ def _same(cfg, **changes):
         assert np.array_equal(q0[k], q1[k]), k
 
 
-# (nside + 6)(nside + 3) rows: less than a block, blocks of 256, 512 and 1024
-# rows on both sides of where one gives way to the next, and just too large
-@pytest.mark.parametrize("nside", [8, 64, 251, 252, 356, 357, 506, 507])
+# (nside + 6)(nside + 3) rows: less than a block; blocks of 256, 512 and 1024
+# rows on both sides of where one gives way to the next; the matrix from
+# memory with 2 to 7 rows a thread on both sides of where they change; and
+# just too large for that
+@pytest.mark.parametrize("nside", [8, 64, 251, 252, 356, 357, 506, 507, 622, 623, 763, 764, 882,
+                                   883, 986, 988, 1081, 1082, 1139, 1142])
 def test_fp64_sizes(require_gpu, nside):
     _same(configs.tank_1m(nside), precision=PREC_FP64)
 
