@@ -776,8 +776,10 @@ int isph_create(const isph_params* prm, int32_t cap, int32_t cap_soil, isph_ctx*
         hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device) ==
             hipSuccess)
         c->cooperative = coop != 0;
+    transfer_attach();
     // the device address of this GPU's isph_probe_noalloc scratch array
     if ((rc = probe_scratch_attach(c))) {
+        transfer_detach();
         (void)hipStreamDestroy(c->stream);
         delete c;
         return rc;
@@ -884,6 +886,7 @@ int isph_destroy(isph_ctx* c) {
             (void)hipEventDestroy(e.b);
         }
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    transfer_detach();
     delete c;
     return ISPH_OK;
 }
@@ -972,35 +975,25 @@ int isph_get_particles(isph_ctx* c, int32_t* n, double* x, double* y, double* vx
                        int32_t* tid, int32_t* flags, int32_t* pid) {
     if (!c) return ISPH_E_ARG;
     if (n) *n = c->n;
-    const int m = c->n;
     StateView& s = c->st[c->cur];
-    const size_t nd = sizeof(double) * m, ni = sizeof(int) * m;
-    auto D2H = hipMemcpyDeviceToHost;
-    std::vector<double2> a;
-    if (x || y) {
-        a.resize(m);
-        HIPCHK(c, hipMemcpyAsync(a.data(), s.pos, sizeof(double2) * m, D2H, c->stream));
-    }
-    std::vector<double2> b;
-    if (vx || vy) {
-        b.resize(m);
-        HIPCHK(c, hipMemcpyAsync(b.data(), s.vel, sizeof(double2) * m, D2H, c->stream));
-    }
-    if (mass) HIPCHK(c, hipMemcpyAsync(mass, s.mass, nd, D2H, c->stream));
-    if (density) HIPCHK(c, hipMemcpyAsync(density, s.rho, nd, D2H, c->stream));
-    if (oden) HIPCHK(c, hipMemcpyAsync(oden, s.oden, nd, D2H, c->stream));
-    if (pressure) HIPCHK(c, hipMemcpyAsync(pressure, s.p, nd, D2H, c->stream));
-    if (tid) HIPCHK(c, hipMemcpyAsync(tid, s.tid, ni, D2H, c->stream));
-    if (flags) HIPCHK(c, hipMemcpyAsync(flags, s.flags, ni, D2H, c->stream));
-    if (pid) HIPCHK(c, hipMemcpyAsync(pid, s.pid, ni, D2H, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < m; ++i) {
-        if (x) x[i] = a[i].x;
-        if (y) y[i] = a[i].y;
-        if (vx) vx[i] = b[i].x;
-        if (vy) vy[i] = b[i].y;
-    }
-    return ISPH_OK;
+    Column col[11];
+    int k = 0;
+    auto want = [&](const void* src, size_t stride, size_t size, void* dst) {
+        if (dst) col[k++] = Column{src, (int)stride, (int)size, dst};
+    };
+    const size_t d = sizeof(double), i = sizeof(int);
+    want(s.pos, 2 * d, d, x);
+    want((double*)s.pos + 1, 2 * d, d, y);
+    want(s.vel, 2 * d, d, vx);
+    want((double*)s.vel + 1, 2 * d, d, vy);
+    want(s.mass, d, d, mass);
+    want(s.rho, d, d, density);
+    want(s.oden, d, d, oden);
+    want(s.p, d, d, pressure);
+    want(s.tid, i, i, tid);
+    want(s.flags, i, i, flags);
+    want(s.pid, i, i, pid);
+    return download(c, c->n, col, k);
 }
 
 int isph_set_soil(isph_ctx* c, int32_t ns, const double* x, const double* y, const double* mass,
@@ -1086,17 +1079,9 @@ int isph_get_field(isph_ctx* c, int32_t f, double* out) {
     bool pair;
     double* p = field_ptr(c, f, &w, &pair, &comp);
     if (!p) return fail(c, ISPH_E_ARG, "unknown field");
-    const int m = c->n;
-    if (pair) {
-        std::vector<double> t(2 * (size_t)m);
-        HIPCHK(c, hipMemcpyAsync(t.data(), p, sizeof(double) * 2 * m, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        for (int i = 0; i < m; ++i) out[i] = t[2 * (size_t)i + comp];
-        return ISPH_OK;
-    }
-    HIPCHK(c, hipMemcpyAsync(out, p, sizeof(double) * w * m, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return ISPH_OK;
+    const int d = (int)sizeof(double);
+    const Column col{p + comp, pair ? 2 * d : d, d, out};
+    return download(c, (int64_t)w * c->n, &col, 1);
 }
 
 int isph_set_field(isph_ctx* c, int32_t f, const double* in) {

@@ -146,6 +146,7 @@ struct isph_ctx {
     } while (0)
 
 namespace isph {
+constexpr int MAX_COLUMNS = 12;  // of one download
 namespace host {
 
 // blocks for n items, at least one: with no particles every per-particle
@@ -165,6 +166,17 @@ int dalloc(isph_ctx* c, T** p, size_t count) {
     HIPCHK(c, hipMemsetAsync(*p, 0, sizeof(T) * (count ? count : 1), c->stream));
     return ISPH_OK;
 }
+// columns of `rows` values to host arrays (isph_transfer.hip); synchronous
+struct Column {
+    const void* src;  // device address of row 0's value
+    int stride;       // bytes from a row's value to the next one's
+    int size;         // of a value: 4 or 8
+    void* dst;        // host array
+};
+int download(isph_ctx* c, int64_t rows, const Column* cols, int ncol);
+void transfer_attach();  // a context lives: the staging memory is kept
+void transfer_detach();
+
 int alloc_state(isph_ctx* c, StateView& s, size_t cap);
 void free_state(StateView& s);
 int copy_state(isph_ctx* c, const StateView& a, const StateView& b, int n);
