@@ -435,15 +435,35 @@ __global__ void __launch_bounds__(MG_CMAX) k_mg_block(MGBlock B, const T* __rest
         w = live ? omega / a[4] : (T)0;
         bc = b[c];
     }
-    // the lower levels' stencils, concatenated as in As (level l from
-    // 9 off[l]; the last level is one cell): every load is issued before the
-    // first store, so the copy costs one memory latency, not one per level
+    // Level 1, where it is smoothed: cell c's stencil stays in registers with
+    // the places of its (clamped) neighbours and, in the upper half words,
+    // their parents on level 2.  A sweep is then nine LDS reads: reading the
+    // stencil from LDS and forming the places again took 0.6 us a barrier
+    // phase for its 160 to 270 cells, twice the top level's.
+    const int nx1 = K > 1 ? B.nx[1] : 1, ny1 = K > 1 ? B.ny[1] : 1, n1 = K > 1 ? nx1 * ny1 : 0;
+    const bool own1 = K > 2 && c < n1;
+    T a1[9], b1 = (T)0;
+    int w1[9], pc1 = 0;
+    if (own1) {
+        const int ny2 = B.ny[2];
+        const int cx = mg_div(c, B.rny[1]), cy = c - cx * ny1;
+#pragma unroll
+        for (int d = 0; d < 9; ++d) {
+            const int ex = mg_clamp(cx + d / 3 - 1, nx1), ey = mg_clamp(cy + d % 3 - 1, ny1);
+            a1[d] = static_cast<const T*>(B.A[1])[(size_t)d * n1 + c];
+            w1[d] = (ex * ny1 + ey) | ((ex >> 1) * ny2 + (ey >> 1)) << 16;
+        }
+        pc1 = (cx >> 1) * ny2 + (cy >> 1);
+    }
+    // the levels below it, concatenated as in As (level l from 9 off[l]; the
+    // last level is one cell): every load is issued before the first store,
+    // so the copy costs one memory latency, not one per level
     constexpr int NST = (9 * MG_CLOW + MG_CMAX - 1) / MG_CMAX;
-    const int tot9 = K > 1 ? 9 * (B.off[K - 1] + 1) : 0;
+    const int lo9 = K > 2 ? 9 * B.off[2] : 0, tot9 = K > 1 ? 9 * (B.off[K - 1] + 1) : 0;
     T st[NST];
 #pragma unroll
     for (int r = 0; r < NST; ++r) {
-        const int e = c + r * MG_CMAX;
+        const int e = lo9 + c + r * MG_CMAX;
         st[r] = (T)0;
         if (e < tot9) {
             const void* src = B.A[1];
@@ -457,13 +477,14 @@ __global__ void __launch_bounds__(MG_CMAX) k_mg_block(MGBlock B, const T* __rest
             st[r] = static_cast<const T*>(src)[e - base];
         }
     }
+    // the exact level's inverse, whether or not it exists, so that its loads
+    // need not wait for the flag (uniform: every thread reads the same)
+    const int D = B.D > 0 && *Aok ? B.D : 0;
+    const int nD = B.D > 0 ? B.nx[B.D] * B.ny[B.D] : 0;
+    for (int e = c; e < nD * nD; e += MG_CMAX) Ai[e] = Ainv[e];
 #pragma unroll
     for (int r = 0; r < NST; ++r)
-        if (c + r * MG_CMAX < tot9) As[c + r * MG_CMAX] = st[r];
-    // the exact level (uniform: every thread reads the same flag)
-    const int D = (B.D > 0 && *Aok) ? B.D : 0;
-    const int nD = D ? B.nx[D] * B.ny[D] : 0;
-    for (int e = c; e < nD * nD; e += MG_CMAX) Ai[e] = Ainv[e];
+        if (lo9 + c + r * MG_CMAX < tot9) As[lo9 + c + r * MG_CMAX] = st[r];
     // LDS keeps what the last kernel on this CU left there: every iterate
     // starts from zero, and a sweep reads the coarser level's iterate only
     // when it applies its correction
@@ -494,49 +515,68 @@ __global__ void __launch_bounds__(MG_CMAX) k_mg_block(MGBlock B, const T* __rest
         }
         __syncthreads();
     };
-    // lower-level sweep: from zero (x1 = omega D^-1 b into parity 1), or from
-    // parity p, with the correction from level l+1 at parity q if corr
+    // level-1 sweep from parity p (with the correction from level 2 at parity
+    // q if corr) and restriction of its residual to level 2
+    auto one_sweep = [&](int p, bool corr, int q) {
+        if (own1) {
+            const T* xc = xl[p];
+            T acc = (T)0;
+            T zi;
+            if (corr) {
+                const T* e = xl[q] + B.off[2];
+                const T f = (T)B.over;
+#pragma unroll
+                for (int d = 0; d < 9; ++d)
+                    acc += a1[d] * (xc[w1[d] & 0xffff] + f * e[w1[d] >> 16]);
+                zi = xc[c] + f * e[pc1];
+            } else {
+#pragma unroll
+                for (int d = 0; d < 9; ++d) acc += a1[d] * xc[w1[d] & 0xffff];
+                zi = xc[c];
+            }
+            const T nv = zi + omega * (b1 - acc) / a1[4];
+            xl[p ^ 1][c] = a1[4] != (T)0 ? nv : (T)0;
+        }
+        __syncthreads();
+    };
+    // lower-level sweep from parity p, with the correction from level l+1 at
+    // parity q if corr.
     // Every LDS load of a sweep is issued before its first use: the diagonal
     // selects the result at the end instead of guarding the loads, and the
     // cell's column comes from B.rny (see mg_div) instead of an integer
     // division; the arithmetic is unchanged.
-    auto low_sweep = [&](int l, int p, bool zero, bool corr, int q) {
+    auto low_sweep = [&](int l, int p, bool corr, int q) {
         const int nx = B.nx[l], ny = B.ny[l], n = nx * ny, o = B.off[l];
         if (c < n) {
             const T* A = As + 9 * o;
             const T dg = A[4 * n + c];
             const T bc = bl[o + c];
-            T nv;
-            if (zero) {
-                nv = omega * bc / dg;
-            } else {
-                const int cx = mg_div(c, B.rny[l]), cy = c - cx * ny;
-                const T* xc = xl[p] + o;
-                T acc = (T)0;
-                T zi;
-                if (corr) {
-                    const int ny2 = B.ny[l + 1];
-                    const T* e = xl[q] + B.off[l + 1];
-                    const T f = (T)B.over;
+            const int cx = mg_div(c, B.rny[l]), cy = c - cx * ny;
+            const T* xc = xl[p] + o;
+            T acc = (T)0;
+            T zi;
+            if (corr) {
+                const int ny2 = B.ny[l + 1];
+                const T* e = xl[q] + B.off[l + 1];
+                const T f = (T)B.over;
 #pragma unroll
-                    for (int d = 0; d < 9; ++d) {
-                        const int ex = mg_clamp(cx + d / 3 - 1, nx);
-                        const int ey = mg_clamp(cy + d % 3 - 1, ny);
-                        acc += A[d * n + c] * (xc[ex * ny + ey] + f * e[(ex >> 1) * ny2 + (ey >> 1)]);
-                    }
-                    zi = xc[c] + f * e[(cx >> 1) * ny2 + (cy >> 1)];
-                } else {
-#pragma unroll
-                    for (int d = 0; d < 9; ++d) {
-                        const int ex = mg_clamp(cx + d / 3 - 1, nx);
-                        const int ey = mg_clamp(cy + d % 3 - 1, ny);
-                        acc += A[d * n + c] * xc[ex * ny + ey];
-                    }
-                    zi = xc[c];
+                for (int d = 0; d < 9; ++d) {
+                    const int ex = mg_clamp(cx + d / 3 - 1, nx);
+                    const int ey = mg_clamp(cy + d % 3 - 1, ny);
+                    acc += A[d * n + c] * (xc[ex * ny + ey] + f * e[(ex >> 1) * ny2 + (ey >> 1)]);
                 }
-                nv = zi + omega * (bc - acc) / dg;
+                zi = xc[c] + f * e[(cx >> 1) * ny2 + (cy >> 1)];
+            } else {
+#pragma unroll
+                for (int d = 0; d < 9; ++d) {
+                    const int ex = mg_clamp(cx + d / 3 - 1, nx);
+                    const int ey = mg_clamp(cy + d % 3 - 1, ny);
+                    acc += A[d * n + c] * xc[ex * ny + ey];
+                }
+                zi = xc[c];
             }
-            xl[zero ? 1 : p ^ 1][o + c] = dg != (T)0 ? nv : (T)0;
+            const T nv = zi + omega * (bc - acc) / dg;
+            xl[p ^ 1][o + c] = dg != (T)0 ? nv : (T)0;
         }
         __syncthreads();
     };
@@ -581,6 +621,29 @@ __global__ void __launch_bounds__(MG_CMAX) k_mg_block(MGBlock B, const T* __rest
         __syncthreads();
     };
 
+    auto one_restrict = [&](int p) {
+        if (own1) {
+            T acc = (T)0;
+#pragma unroll
+            for (int d = 0; d < 9; ++d) acc += a1[d] * xl[p][w1[d] & 0xffff];
+            rt[c] = b1 - acc;
+        }
+        __syncthreads();
+        const int ny2 = B.ny[2];
+        if (c < B.nx[2] * ny2) {
+            const int X = mg_div(c, B.rny[2]), Y = c - X * ny2;
+            T s = (T)0;
+            for (int u = 0; u < 2; ++u)
+                for (int v = 0; v < 2; ++v) {
+                    const int cx = 2 * X + u, cy = 2 * Y + v;
+                    if (cx < nx1 && cy < ny1) s += rt[cx * ny1 + cy];
+                }
+            bl[B.off[2] + c] = s;
+            if (2 < Lx) zero_sweep(2, c, s);
+        }
+        __syncthreads();
+    };
+
     if (K == 1) {  // a single cell: exact
         if (own) x[c] = live ? bc / a[4] : (T)0;
         return;
@@ -609,16 +672,25 @@ __global__ void __launch_bounds__(MG_CMAX) k_mg_block(MGBlock B, const T* __rest
                         if (cx < B.nx[0] && cy < ny0) s += rt[cx * ny0 + cy];
                     }
                 bl[B.off[1] + c] = s;
-                if (1 < Lx) zero_sweep(1, c, s);
+                b1 = s;
+                if (1 < Lx) xl[1][c] = a1[4] != (T)0 ? omega * s / a1[4] : (T)0;
             }
             __syncthreads();
         }
         // down the lower levels: smoothing (the sweep from zero was made with
         // the restriction into the level), restriction
-        for (int l = 1; l < Lx; ++l) {
+        if (1 < Lx) {
             int p = 1;
             for (int s = 1; s < nu; ++s) {
-                low_sweep(l, p, false, false, 0);
+                one_sweep(p, false, 0);
+                p ^= 1;
+            }
+            one_restrict(p);
+        }
+        for (int l = 2; l < Lx; ++l) {
+            int p = 1;
+            for (int s = 1; s < nu; ++s) {
+                low_sweep(l, p, false, 0);
                 p ^= 1;
             }
             low_restrict(l, p);
@@ -627,6 +699,7 @@ __global__ void __launch_bounds__(MG_CMAX) k_mg_block(MGBlock B, const T* __rest
             const int o = B.off[D];
             if (c < nD) {
                 T acc = (T)0;
+#pragma unroll 8
                 for (int j = 0; j < nD; ++j) acc += Ai[j * nD + c] * bl[o + j];
                 xl[1][o + c] = acc;
             }
@@ -641,12 +714,22 @@ __global__ void __launch_bounds__(MG_CMAX) k_mg_block(MGBlock B, const T* __rest
         }
         // up: correction folded into the first post-smoothing sweep
         int q = 1;  // parity of level l+1's iterate
-        for (int l = Lx - 1; l >= 1; --l) {
+        for (int l = Lx - 1; l >= 2; --l) {
             int p = nu & 1;
-            low_sweep(l, p, false, true, q);
+            low_sweep(l, p, true, q);
             p ^= 1;
             for (int s = 1; s < nu; ++s) {
-                low_sweep(l, p, false, false, 0);
+                low_sweep(l, p, false, 0);
+                p ^= 1;
+            }
+            q = p;
+        }
+        if (1 < Lx) {
+            int p = nu & 1;
+            one_sweep(p, true, q);
+            p ^= 1;
+            for (int s = 1; s < nu; ++s) {
+                one_sweep(p, false, 0);
                 p ^= 1;
             }
             q = p;
