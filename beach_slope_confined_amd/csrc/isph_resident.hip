@@ -22,10 +22,16 @@
 // expressions, so only v and t go through memory, 8 bytes a row each.  The
 // exchanges are the only grid-wide synchronisations (isph_gridsync.h).
 //
-// What bounds it: the chain of three exchanges (2 us each for the words' way to
-// the leader and back, about 1 us for the sums on either side), two products
-// from LDS (0.5 us each) and the halo reads (0.8 us).  Measured per iteration,
-// launched kernels and here: 30 and 12.8 us at 36.6k rows, 32 and 13 us at 87k.
+// The first entries of a row's matrix are in registers, the next in LDS, and
+// only where a thread has 128 registers (blocks of 1024 rows) a few stay in
+// memory.
+//
+// What bounds it: the chain of three exchanges (2.3 us each: the words' way to
+// the leader and back, the sums on either side), then two products (0.5 us),
+// the halo reads (0.4 us) and the wait for the stores.  Measured per
+// iteration, launched kernels and here: 30 and 10.3 us at 36.6k rows, 32 and
+// 11.7 us at 87k, 44 and 19 us at 255k.  Values and places in LDS instead of
+// registers, with the diagonal tested at every entry, made a product 1.3 us.
 //
 // The arithmetic is the launched kernels', term for term: the same row sums,
 // the same reduction tree (wave butterfly, four waves of 256 rows, then
@@ -47,10 +53,11 @@ constexpr int RESIDENT_M = 3;          // halo rows a thread carries
 constexpr int RESIDENT_SPAN = 16384;   // rows from a window's first to its last, at most
 constexpr int RESIDENT_WORDS = RESIDENT_SPAN / 32;
 
-// entries of a row loaded together (with 1024 threads a thread has 128 registers)
+// entries of a row kept in registers (a thread has 512, 256 or 128 of them with
+// blocks of 256, 512 or 1024)
 template <int G>
-struct ResidentUnroll {
-    static constexpr int value = G == 4 ? 6 : 8;
+struct ResidentRegs {
+    static constexpr int value = G == 4 ? 8 : 24;
 };
 
 // The block's window: a bit per row of [base, base + RESIDENT_SPAN), and the
@@ -63,52 +70,114 @@ struct Window {
     }
 };
 
-// One row times the vector in LDS, as spmv_row (unit diagonal at dp) or, for
-// FP32 values with FP64 vectors, as spmv_row_diff (FP64 row sum si).  Entries
-// k < kl come from LDS (every STRIDE-th element, places in the window), a
-// group that reaches past them from the matrix in memory (columns).  Indices
-// are clamped to the row's last entry; the sum takes the row's own entries
-// only, in order.
-template <int U, bool DIFF, int STRIDE, class TV, class TX>
-__device__ __forceinline__ TX resident_row(int i, int c, int dp, double si, int kl, int base,
-                                           const Window& W, const TV* lv,
-                                           const unsigned short* lj, const short* nbr, const TV* val,
-                                           size_t ld, TX xi, const TX* win) {
-    TX s = (TX)0;
-    for (int k = 0; k < c; k += U) {
-        TV v[U];
-        TX x[U];
-        int j[U];
-        if (min(k + U, c) <= kl) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int e = min(k + u, c - 1) * STRIDE;
-                j[u] = lj[e];
-                v[u] = lv[e];
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const size_t o = (size_t)min(k + u, c - 1) * ld + i;
-                j[u] = col_of(nbr[o], i);
-                v[u] = val[o];
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) j[u] = W.place(j[u] - base);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = win[j[u]];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (!DIFF && k + u == dp && k + u < c) s = s + xi;
-            const TX t = DIFF ? s + (TX)v[u] * (x[u] - xi) : s + (TX)v[u] * x[u];
-            s = k + u < c ? t : s;
-        }
+// A row's entries in column order, as spmv_row takes them: the unit diagonal
+// is an entry of its own, 1 at position dp (1 x is x, so the sum is the same),
+// and for FP32 values with FP64 vectors (spmv_row_diff) there is none.  The
+// first NREG are in registers, the next kl in LDS (every STRIDE-th element),
+// the rest in memory.  Rows are padded with 0 times their own x: a sum that
+// starts from +0 is never -0, so adding 0 changes nothing.
+template <bool DIFF, int NREG, int STRIDE, class TV, class TX>
+struct ResidentRow {
+    int i, c, dp, len, own;    // row, list entries, diagonal, entries, own byte offset in the window
+    int wlen;                  // longest row of the wave
+    double si;
+    TV v[NREG];
+    unsigned int off[NREG / 2];  // byte offsets in the window, two a word
+    const TV* lv;
+    const unsigned short* lo;
+
+    // entry e of the list with the diagonal: its place in the matrix, or -1
+    __device__ __forceinline__ int source(int e) const {
+        return DIFF ? e : e < dp ? e : e == dp ? -1 : e - 1;
     }
-    if (DIFF) return (TX)si * xi + s;
-    if (dp == c) s = s + xi;
-    return s;
-}
+    __device__ __forceinline__ void load(const KrylovArgs<TV, TX, short>& a, const Window& W,
+                                         int base, int kl, TV* lvw, unsigned short* low) {
+        auto entry = [&](int e, TV& val, unsigned int& o) {
+            val = (TV)0;
+            o = own;
+            if (e < len) {
+                const int k = source(e);
+                if (k < 0) {
+                    val = (TV)1;
+                } else {
+                    val = a.val[(size_t)k * a.ld + i];
+                    o = W.place(i + (int)a.nbr[(size_t)k * a.ld + i] - base) * (int)sizeof(TX);
+                }
+            }
+        };
+#pragma unroll
+        for (int e = 0; e < NREG; e += 2) {
+            unsigned int o0, o1;
+            entry(e, v[e], o0);
+            entry(e + 1, v[e + 1], o1);
+            off[e / 2] = o0 | o1 << 16;
+        }
+        for (int e = 0; e < kl && NREG + e < ((len + 3) & ~3); ++e) {
+            TV val;
+            unsigned int o;
+            entry(NREG + e, val, o);
+            lvw[e * STRIDE] = val;
+            low[e * STRIDE] = (unsigned short)o;
+        }
+        lv = lvw;
+        lo = low;
+        int m = len;
+        for (int s = 1; s < 64; s <<= 1) m = max(m, __shfl_xor(m, s, 64));
+        wlen = __builtin_amdgcn_readfirstlane(m);
+    }
+    __device__ __forceinline__ TX times(const KrylovArgs<TV, TX, short>& a, const Window& W,
+                                        int base, int kl, const TX* win, TX xi) const {
+        const char* w = reinterpret_cast<const char*>(win);
+        auto at = [&](unsigned int o) { return *reinterpret_cast<const TX*>(w + o); };
+        auto add = [&](TX s, TV val, TX x) {
+            return DIFF ? s + (TX)val * (x - xi) : s + (TX)val * x;
+        };
+        TX s = (TX)0;
+#pragma unroll
+        for (int e = 0; e < NREG; e += 8) {
+            if (e >= wlen) break;  // the same in the whole wave
+            TX x[8];
+#pragma unroll
+            for (int u = 0; u < 8; u += 2) {
+                x[u] = at(off[(e + u) / 2] & 0xffff);
+                x[u + 1] = at(off[(e + u) / 2] >> 16);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s = add(s, v[e + u], x[u]);
+        }
+        if (wlen > NREG) {
+            const int in_lds = min(len - NREG, kl);
+            for (int e = 0; e < in_lds; e += 4) {
+                TV val[4];
+                TX x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    val[u] = lv[(e + u) * STRIDE];
+                    x[u] = at(lo[(e + u) * STRIDE]);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) s = add(s, val[u], x[u]);
+            }
+            for (int e = NREG + kl; e < len; e += 4) {
+                TV val[4];
+                TX x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int k = source(min(e + u, len - 1));
+                    const size_t o = (size_t)max(k, 0) * a.ld + i;
+                    val[u] = k < 0 ? (TV)1 : a.val[o];
+                    x[u] = k < 0 ? xi : win[W.place(i + (int)a.nbr[o] - base)];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const TX t = add(s, val[u], x[u]);
+                    s = e + u < len ? t : s;
+                }
+            }
+        }
+        return DIFF ? (TX)si * xi + s : s;
+    }
+};
 
 // A worker's part of an exchange: the block's partials in the launched
 // kernels' tree, published by one thread.  STORED: the waves have stored
@@ -143,64 +212,53 @@ __device__ __forceinline__ void publish_sums(const GridSync& gs, double (*wsum)[
     }
 }
 
-// The leader: finishes each exchange's reduction and the solver scalars, and
-// broadcasts the scalar that the workers wait for.
+// The leader, one wave: finishes each exchange's reduction and the solver
+// scalars, and broadcasts the scalar that the workers wait for.  Lane l takes
+// the parts l + 64 m.  64 / G parts are a wave of k_finish's tree, so the sum
+// over the lanes of one m covers G of its waves, in its order: the butterfly's
+// last log2(G) steps are the first levels of the tree over the waves.
 template <int G>
-__device__ __forceinline__ void resident_leader(const GridSync& gs, double (*red)[16], int* lost,
-                                                int nw, SolverScalars* sc, const SolveCtl& ctl,
-                                                int maxiter) {
-    constexpr int PER = 64 / G;  // workers per wave of k_finish's tree
-    if (threadIdx.x >= 256) return;
+__device__ __forceinline__ void resident_leader(const GridSync& gs, int nw, SolverScalars* sc,
+                                                const SolveCtl& ctl, int maxiter) {
+    constexpr int NP = GS_MAXB / 64;
     const int t = threadIdx.x;
-    if (t < 32) red[t >> 4][t & 15] = 0.0;
-    if (t == 0) *lost = 0;
-    __syncthreads();
+    if (t >= 64) return;
     SolverScalars s = *sc;
-    auto tree = [](const double* r) {
-        double a[8];
+    double a[NP] = {}, b[NP] = {};
+    auto collect = [&](uint32_t e, bool two) {
+        const bool ok = t >= nw || gs_collect<NP>(gs, e, t, 64, nw, two, a, b);
+        if (!__all(ok)) {
+            if (t == 0) atomicOr(gs.err, ERR_SYNC);
+            return false;
+        }
+        return true;
+    };
+    // k_finish's remaining waves are 0
+    auto total = [](const double* p) {
+        double q[NP];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) a[k] = r[2 * k] + r[2 * k + 1];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) a[k] = a[2 * k] + a[2 * k + 1];
-        return (a[0] + a[1]) + (a[2] + a[3]);
+        for (int m = 0; m < NP; ++m) q[m] = lanes_sum<64>(p[m]);
+        return ((q[0] + q[1]) + (q[2] + q[3])) + 0.0;
     };
     // epoch 1: do all blocks' windows fit?
     uint32_t e = 1;
-    {
-        double a = 0.0, b = 0.0;
-        if (t < nw && !gs_collect<1>(gs, e, t, 0, nw, false, &a, &b)) *lost = 1;
-        if (a != 0.0) *lost = 2;
-    }
-    __syncthreads();
-    const int refused = *lost;
+    if (!collect(e, false)) return;
+    const int refused = total(a) != 0.0;
     gs_broadcast(gs, e, 0.0, refused);
     if (refused) {
-        if (t == 0) refused == 1 ? atomicOr(gs.err, ERR_SYNC) : atomicOr(gs.state, GS_REFUSED);
+        if (t == 0) atomicOr(gs.state, GS_REFUSED);
         return;
     }
     for (int it = 0; it < maxiter; ++it) {
-#pragma unroll 1
-        for (int kind = FIN_ALPHA; kind <= FIN_BETA; ++kind) {
-            ++e;
-            const bool two = kind != FIN_ALPHA;
-            double a = 0.0, b = 0.0;
-            if (t < nw && !gs_collect<1>(gs, e, t, 0, nw, two, &a, &b)) *lost = 1;
-            a = lanes_sum<PER>(a);
-            b = lanes_sum<PER>(b);
-            if (t % PER == 0) {
-                red[0][t / PER] = a;
-                red[1][t / PER] = b;
-            }
-            __syncthreads();
-            if (*lost) {
-                if (t == 0) atomicOr(gs.err, ERR_SYNC);
-                return;
-            }
-            finish_update(kind, tree(red[0]), tree(red[1]), s, ctl);
-            gs_broadcast(gs, e, kind == FIN_ALPHA ? s.alpha : kind == FIN_OMEGA ? s.wi : s.betas,
-                         s.done);
-            __syncthreads();  // red is read before the next exchange writes it
-        }
+        if (!collect(++e, false)) return;
+        finish_update(FIN_ALPHA, total(a), 0.0, s, ctl);
+        gs_broadcast(gs, e, s.alpha, 0);
+        if (!collect(++e, true)) return;
+        finish_update(FIN_OMEGA, total(a), total(b), s, ctl);
+        gs_broadcast(gs, e, s.wi, 0);
+        if (!collect(++e, true)) return;
+        finish_update(FIN_BETA, total(a), total(b), s, ctl);
+        gs_broadcast(gs, e, s.betas, s.done);
         if (s.done) break;
     }
     if (t == 0) *sc = s;
@@ -215,14 +273,14 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
     constexpr bool DIFF = std::is_same<TV, float>::value && std::is_same<TX, double>::value;
     constexpr int R = BLOCK * G;
     constexpr int M = RESIDENT_M;
-    constexpr int U = ResidentUnroll<G>::value;
+    constexpr int NREG = ResidentRegs<G>::value;
     extern __shared__ double dyn[];
     __shared__ double sums[2][16];
     __shared__ Window W;
     __shared__ int jlo, jhi, total;
     const int nw = gridDim.x - 1;
     if ((int)blockIdx.x == nw) {
-        resident_leader<G>(gs, sums, &jlo, nw, sc, ctl, maxiter);
+        resident_leader<G>(gs, nw, sc, ctl, maxiter);
         return;
     }
     const int block = xcd_tile(blockIdx.x, nw);
@@ -295,12 +353,14 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
     TX* win = reinterpret_cast<TX*>(dyn);
     TV* lv = reinterpret_cast<TV*>(win + (M + 1) * R) + t;
     unsigned short* lj = reinterpret_cast<unsigned short*>(lv - t + (size_t)kl * R) + t;
-    if (own)
-        for (int k = 0; k < min(c, kl); ++k) {
-            lv[k * R] = a.val[(size_t)k * a.ld + i];
-            lj[k * R] =
-                (unsigned short)W.place(col_of(a.nbr[(size_t)k * a.ld + i], i) - base);
-        }
+    ResidentRow<DIFF, NREG, R, TV, TX> row;
+    row.i = i;
+    row.c = c;
+    row.dp = dp;
+    row.len = own ? c + (DIFF ? 0 : 1) : 0;
+    row.own = (nl + t) * (int)sizeof(TX);
+    row.si = si;
+    row.load(a, W, base, kl, lv, lj);
     // halo row h is the window's h-th row that is not the block's own; the
     // list of them passes through the window's memory
     unsigned short* list = reinterpret_cast<unsigned short*>(dyn);
@@ -332,6 +392,10 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
     }
     TX* vout = a.si;   // the launched kernels' s and t vectors carry v and t
     TX* tout = a.mm2;
+    // 32-bit byte offsets: one register an address
+    auto at = [](TX* v, int j) {
+        return reinterpret_cast<TX*>(reinterpret_cast<char*>(v) + (unsigned int)j * (unsigned int)sizeof(TX));
+    };
     coef = sc->betas;
     bool ok = true;
     for (int it = 0; it < maxiter; ++it) {
@@ -349,8 +413,8 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         __syncthreads();
         TX v = (TX)0;
         if (own) {
-            v = resident_row<U, DIFF, R>(i, c, dp, si, kl, base, W, lv, lj, a.nbr, a.val, a.ld, p, win);
-            gs_store(vout + i, v);
+            v = row.times(a, W, base, kl, win, p);
+            gs_store(at(vout, i), v);
         }
         publish_sums<G, false, true>(gs, sums, ++e, block, own ? (double)v * (double)rhat : 0.0,
                                      0.0);
@@ -361,7 +425,7 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         if (own) win[nl + t] = sv;
 #pragma unroll
         for (int m = 0; m < M; ++m)
-            if (hj[m] >= 0) hv[m] = gs_load(vout + hj[m]);
+            if (hj[m] >= 0) hv[m] = gs_load(at(vout, hj[m]));
 #pragma unroll
         for (int m = 0; m < M; ++m)
             if (hj[m] >= 0) {
@@ -371,8 +435,8 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         __syncthreads();
         TX tv = (TX)0;
         if (own) {
-            tv = resident_row<U, DIFF, R>(i, c, dp, si, kl, base, W, lv, lj, a.nbr, a.val, a.ld, sv, win);
-            gs_store(tout + i, tv);
+            tv = row.times(a, W, base, kl, win, sv);
+            gs_store(at(tout, i), tv);
         }
         publish_sums<G, true, true>(gs, sums, ++e, block, own ? (double)tv * (double)sv : 0.0,
                                     own ? (double)tv * (double)tv : 0.0);
@@ -382,7 +446,7 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         TX ht[M];
 #pragma unroll
         for (int m = 0; m < M; ++m)
-            ht[m] = hj[m] >= 0 ? gs_load(tout + hj[m]) : (TX)0;
+            ht[m] = hj[m] >= 0 ? gs_load(at(tout, hj[m])) : (TX)0;
         x = (x + alpha * p) + w * sv;
         r = sv - w * tv;
         q = p - w * v;
@@ -420,10 +484,11 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
     constexpr int R = BLOCK * G;
     const int blocks = (nblk(c->n) + G - 1) / G + 1;
     if (blocks > c->cus) return ISPH_OK;
-    // the gathered window, then as many entries of each row as fit
+    // the gathered window, then as many of each row's further entries as fit
     constexpr size_t win = sizeof(TX) * (RESIDENT_M + 1) * R;
     constexpr size_t per = (sizeof(TV) + sizeof(unsigned short)) * R;
-    const int kl = (int)std::min<size_t>((size_t)c->prm.max_nbr, (RESIDENT_LDS - win) / per);
+    const size_t most = (size_t)std::max(c->prm.max_nbr + 4 - ResidentRegs<G>::value, 0);
+    const int kl = (int)std::min(most, (RESIDENT_LDS - win) / per) & ~3;  // taken in fours
     const size_t lds = win + per * kl;
     KrylovArgs<TV, TX, short> a = ka;
     GridSync gs{c->gs_words, c->err, c->err + 1, GS_MAXB};
