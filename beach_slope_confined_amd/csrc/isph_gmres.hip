@@ -17,9 +17,11 @@
 // norm, iteration limit, end of the restart cycle.
 //
 // One Arnoldi step j (classical Gram-Schmidt applied twice, CGS2):
-//   k_gm_arnoldi  v_j = u / beta, w = A v_j, partials (v_i, w), i <= j
+//   k_gm_arnoldi  v_j = u / beta, w = A v_j
+//   k_gm_dots     partials (v_i, w), i <= j
 //   k_gm_fin      h1_i, one block per i, k_finish's tree
-//   k_gm_orth     u = w - sum_i h1_i v_i (i ascending), partials (v_i, u)
+//   k_gm_orth     u = w - sum_i h1_i v_i (i ascending)
+//   k_gm_dots     partials (v_i, u)
 //   k_gm_fin      h2_i
 //   k_gm_orth2    u = u - sum_i h2_i v_i, partial (u, u)
 //   k_gm_givens   one thread: column h1 + h2, the earlier rotations, a new
@@ -40,8 +42,8 @@ namespace isph {
 constexpr int GM_DEFAULT_M = 150;       // MKL's default restart length and limit
 constexpr int GM_MAXM = 512;            // longest restart cycle accepted
 constexpr double GM_ZERO_NORM = 1e-12;  // dpar(8)
-constexpr int GM_CHUNK = 8;             // basis vectors per block reduction round
-constexpr int GM_SUB = 8;               // basis vectors loaded ahead in a subtraction
+constexpr int GM_CHUNK = 8;             // basis vectors of a block of dots
+constexpr int GM_SUB = 16;              // basis vectors loaded ahead in a subtraction
 constexpr int GM_BATCH = 8;             // Arnoldi steps enqueued between host reads
 
 enum { GM_RUN = 0, GM_CONV = 1, GM_HAPPY = 2, GM_CYCLE = 3, GM_MAXIT = 4, GM_FAIL = 5 };
@@ -82,23 +84,35 @@ __device__ __forceinline__ void block_sum_k(double (&v)[K]) {
     for (int k = 0; k < K; ++k) v[k] = (red[k][0] + red[k][1]) + (red[k][2] + red[k][3]);
 }
 
-// partials (v_i, w) for i = 0..j into part[i * nbp + lb]; rows past n add 0
-__device__ __forceinline__ void gm_dots(bool valid, int r, int j, const double* __restrict__ V,
-                                        size_t cap, double w, double* __restrict__ part,
-                                        int nbp, int lb) {
-    for (int i0 = 0; i0 <= j; i0 += GM_CHUNK) {
-        double v[GM_CHUNK];
+// Partials (v_i, w) for i <= j into part[i * nbp + lb]; rows past n add 0.
+// A block takes 256 rows of GM_CHUNK basis vectors: the products of different
+// vectors are independent, so the grid is (j + 1) / GM_CHUNK times the rows'
+// and the chip is full however few rows there are.  With the dots as a loop
+// over the chunks in the kernels that make w and u (one block reduction between
+// a chunk's loads and the next's) those took 38.5 and 38 us at 86k rows, mean
+// of 150 columns; they take 7.7 and 9.9 now and this kernel 9.6 for each.  A
+// column in all: 120 -> 68 us at 93k rows, 243 -> 160 at 319k, 651 -> 501 at
+// 1.01M (whole step over its 150 columns), where the basis comes from HBM.
+__global__ void __launch_bounds__(BLOCK) k_gm_dots(int n, int j, const double* __restrict__ V,
+                                                   size_t cap, const double* __restrict__ w,
+                                                   const GmState* st, double* __restrict__ part) {
+    const int done = st->done;  // tested once the loads are requested
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int r = lb * BLOCK + threadIdx.x, i0 = blockIdx.y * GM_CHUNK;
+    const bool valid = r < n;
+    const double wr = valid ? w[r] : 0.0;
+    double v[GM_CHUNK];
 #pragma unroll
-        for (int k = 0; k < GM_CHUNK; ++k) {
-            const int i = i0 + k;
-            v[k] = (valid && i <= j) ? V[(size_t)i * cap + r] * w : 0.0;
-        }
-        block_sum_k<GM_CHUNK>(v);
-        if (threadIdx.x == 0)
+    for (int k = 0; k < GM_CHUNK; ++k)
+        v[k] = (valid && i0 + k <= j) ? V[(size_t)(i0 + k) * cap + r] : 0.0;
+    if (done) return;
 #pragma unroll
-            for (int k = 0; k < GM_CHUNK; ++k)
-                if (i0 + k <= j) part[(size_t)(i0 + k) * nbp + lb] = v[k];
-    }
+    for (int k = 0; k < GM_CHUNK; ++k) v[k] = (valid && i0 + k <= j) ? v[k] * wr : 0.0;
+    block_sum_k<GM_CHUNK>(v);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < GM_CHUNK; ++k)
+            if (i0 + k <= j) part[(size_t)(i0 + k) * gridDim.x + lb] = v[k];
 }
 
 // x - h_0 v_0 - h_1 v_1 - ... - h_j v_j at row r, subtracted in order; the
@@ -162,26 +176,21 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_gm_start(int nbp, const double* _
         st->done = GM_RUN;
 }
 
-// v_j = u / beta (stored), w = A v_j, partials (v_i, w) for i <= j
+// v_j = u / beta (stored), w = A v_j
 template <class TI>
 __global__ void __launch_bounds__(BLOCK) k_gm_arnoldi(GmMat<TI> A, int j, double* __restrict__ V,
                                                       size_t cap, const double* __restrict__ u,
-                                                      double* __restrict__ w, const GmState* st,
-                                                      double* __restrict__ part) {
+                                                      double* __restrict__ w, const GmState* st) {
     if (st->done) return;
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int r = lb * BLOCK + threadIdx.x;
-    const bool valid = r < A.n;
     const double beta = st->beta;
-    double wr = 0.0;
-    if (valid) {
+    if (r < A.n) {
         const double vr = u[r] / beta;
         V[(size_t)j * cap + r] = vr;
         auto vj = [&](int c) { return u[c] / beta; };
-        wr = spmv_row<double, double, TI>(r, A.cnt[r], A.dpos[r], A.nbr, A.val, A.ld, vr, vj);
-        w[r] = wr;
+        w[r] = spmv_row<double, double, TI>(r, A.cnt[r], A.dpos[r], A.nbr, A.val, A.ld, vr, vj);
     }
-    gm_dots(valid, r, j, V, cap, wr, part, gridDim.x, lb);
 }
 
 // out[i] = the finished sum of partial column i (one block per column)
@@ -192,22 +201,15 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_gm_fin(int nbp, const double* __r
     if (threadIdx.x == 0) out[blockIdx.x] = t;
 }
 
-// u = w - sum_i h_i v_i, partials (v_i, u) for the second pass
+// u = w - sum_i h_i v_i
 __global__ void __launch_bounds__(BLOCK) k_gm_orth(int n, int j, const double* __restrict__ V,
                                                    size_t cap, const double* __restrict__ w,
                                                    const double* __restrict__ h,
-                                                   double* __restrict__ u, const GmState* st,
-                                                   double* __restrict__ part) {
+                                                   double* __restrict__ u, const GmState* st) {
     if (st->done) return;
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int r = lb * BLOCK + threadIdx.x;
-    const bool valid = r < n;
-    double x = 0.0;
-    if (valid) {
-        x = gm_subtract(w[r], r, j, V, cap, h);
-        u[r] = x;
-    }
-    gm_dots(valid, r, j, V, cap, x, part, gridDim.x, lb);
+    if (r < n) u[r] = gm_subtract(w[r], r, j, V, cap, h);
 }
 
 // u = u - sum_i h2_i v_i, partial (u, u)
@@ -291,14 +293,46 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_gm_givens(int j, int m, int maxit
         st->done = GM_CYCLE;
 }
 
-// y = R^-1 g on the first k columns (back substitution, one thread)
-__global__ void k_gm_lsq(int k, int m, const double* __restrict__ R, const double* __restrict__ g,
-                         double* __restrict__ y) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+// y = R^-1 g on the first k columns: one wave.  Row i subtracts its products
+// with l ascending, a serial chain; its lanes make the products, and the next
+// row's entries are requested before the chain starts, so the chain alone is
+// left (one thread that also fetched and multiplied: 224 us at 150 columns).
+__global__ void __launch_bounds__(64) k_gm_lsq(int k, int m, const double* __restrict__ R,
+                                               const double* __restrict__ g,
+                                               double* __restrict__ y) {
+    __shared__ double ys[GM_MAXM], prod[GM_MAXM];
+    constexpr int Q = GM_MAXM / 64;
+    const int t = threadIdx.x;
+    const size_t ld = m + 1;
+    double row[Q], diag = 0.0, rhs = 0.0;
+    auto request = [&](int i) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int l = q * 64 + t;
+            row[q] = (l > i && l < k) ? R[l * ld + i] : 0.0;
+        }
+        diag = R[i * ld + i];
+        rhs = g[i];
+    };
+    request(k - 1);
     for (int i = k - 1; i >= 0; --i) {
-        double s = g[i];
-        for (int l = i + 1; l < k; ++l) s = s - R[(size_t)l * (m + 1) + i] * y[l];
-        y[i] = s / R[(size_t)i * (m + 1) + i];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int l = q * 64 + t;
+            if (l > i && l < k) prod[l] = row[q] * ys[l];
+        }
+        double s = rhs;
+        const double d = diag;
+        __syncthreads();
+        if (i > 0) request(i - 1);
+#pragma unroll 8
+        for (int l = i + 1; l < k; ++l) s = s - prod[l];
+        s = s / d;
+        if (t == 0) {
+            ys[i] = s;
+            y[i] = s;
+        }
+        __syncthreads();
     }
 }
 
@@ -390,11 +424,12 @@ static int gm_run(isph_ctx* c, const GmMat<TI>& A, double* x, int m, bool& conve
             const int nb = std::min(GM_BATCH, m - h.j);
             for (int b = 0; b < nb; ++b) {
                 const int j = h.j + b;
-                k_gm_arnoldi<TI><<<grid, BLOCK, 0, c->stream>>>(A, j, d->V, cap, d->u, d->w, d->st,
-                                                                d->part);
+                const dim3 dots(grid, j / GM_CHUNK + 1);
+                k_gm_arnoldi<TI><<<grid, BLOCK, 0, c->stream>>>(A, j, d->V, cap, d->u, d->w, d->st);
+                k_gm_dots<<<dots, BLOCK, 0, c->stream>>>(n, j, d->V, cap, d->w, d->st, d->part);
                 k_gm_fin<<<j + 1, FIN_BLOCK, 0, c->stream>>>(grid, d->part, d->h1, d->st);
-                k_gm_orth<<<grid, BLOCK, 0, c->stream>>>(n, j, d->V, cap, d->w, d->h1, d->u, d->st,
-                                                         d->part);
+                k_gm_orth<<<grid, BLOCK, 0, c->stream>>>(n, j, d->V, cap, d->w, d->h1, d->u, d->st);
+                k_gm_dots<<<dots, BLOCK, 0, c->stream>>>(n, j, d->V, cap, d->u, d->st, d->part);
                 k_gm_fin<<<j + 1, FIN_BLOCK, 0, c->stream>>>(grid, d->part, d->h2, d->st);
                 k_gm_orth2<<<grid, BLOCK, 0, c->stream>>>(n, j, d->V, cap, d->h2, d->u, d->st,
                                                           d->part);
