@@ -196,22 +196,27 @@ __global__ void k_mg_galerkin(int nx, int ny, const T* __restrict__ A, int nx2, 
 // ---------------------------------------------------------------------------
 // V-cycle kernels (value type T: float for MIXED_MG, double for FP64_MG)
 // ---------------------------------------------------------------------------
-// Level 0 down.  The right-hand side b is formed from the outer pairs:
-// MODE 0: b = p = r + beta q (r on a restart), from rq = (r, q);
-// MODE 1: b = s = r - alpha v, from rv = (r, v).  b goes to bout (FP64, the
-// outer recurrences need it).  Without pre-smoothing the particle iterate is
-// 0 and its residual is b itself, r0 = (T) b.
+// Level 0 down: the V-cycle's right-hand side.
+// MODE 0: b = p = r + beta q, q = p - omega v (p = r on a restart);
+// MODE 1: b = s = r - alpha v.
+// b goes to bout (FP64, the outer recurrences need it; MODE 0 updates p in
+// place).  Without pre-smoothing the particle iterate is 0 and its residual is
+// b itself, r0 = (T) b, which is also what the last sweep reads.
 template <class T, int MODE, bool FIRST>
-__global__ void k_mg_bpoint(int n, const double2* __restrict__ pairs, const SolverScalars* sc,
-                            double* __restrict__ bout, T* __restrict__ r0) {
-    // the flag, the coefficient and the pair are requested together
+__global__ void k_mg_bpoint(int n, const double* __restrict__ r, const double* __restrict__ v,
+                            const SolverScalars* sc, double* __restrict__ bout,
+                            T* __restrict__ r0) {
+    // the flag, the coefficients and the operands are requested together
     const int done = sc->done;
-    const double coef = MODE == 0 ? sc->betas : sc->alpha;
+    const double coef = MODE == 0 ? sc->betas : sc->alpha, w = sc->wi;
     int i = blockIdx.x * BLOCK + threadIdx.x;
     if (i >= n) return;
-    const double2 u = pairs[i];
+    const double ri = r[i];
+    const double vi = FIRST ? 0.0 : v[i], pi = MODE == 0 && !FIRST ? bout[i] : 0.0;
     if (done) return;
-    const double bi = MODE == 0 ? (FIRST ? u.x : u.x + coef * u.y) : u.x - coef * u.y;
+    double bi = ri;
+    if (MODE == 0 && !FIRST) bi = ri + coef * (pi - w * vi);
+    if (MODE == 1) bi = ri - coef * vi;
     bout[i] = bi;
     r0[i] = (T)bi;
 }
@@ -1008,9 +1013,9 @@ template <class T>
 __global__ void __launch_bounds__(BLOCK) k_mg_fine_up(int n, size_t ld, int ny,
                                                       const int* __restrict__ cell,
                                                       const T* __restrict__ p9,
-                                                      const double* __restrict__ b,
+                                                      const T* __restrict__ b,
                                                       const T* __restrict__ e1, float over,
-                                                      double* __restrict__ out,
+                                                      T* __restrict__ out,
                                                       const SolverScalars* sc) {
     const int done = sc->done;  // tested once the row's cell is requested
     int i = xcd_tile(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x;
@@ -1027,17 +1032,25 @@ __global__ void __launch_bounds__(BLOCK) k_mg_fine_up(int n, size_t ld, int ny,
     T acc = (T)0;
 #pragma unroll
     for (int d = 0; d < 9; ++d) acc += pv[d] * zv[d];
-    out[i] = (double)(zv[4] + mg_omega<T>() * ((T)b[i] - acc));
+    out[i] = zv[4] + mg_omega<T>() * (b[i] - acc);
 }
 
 // ---------------------------------------------------------------------------
 // outer BiCGSTAB kernels (FP64 vectors, partials per XCD-mapped block)
+// These are bound by the bytes of their vectors and matrix, so no vector is
+// moved that can be left where it is: r stays in the array of the true
+// residual, v is written alone (as pairs (r, v) and (r, q) for a gather that
+// this solve does not have, k_mg_v and k_mg_x moved r and q along), q is formed
+// where p is, p^ and s^ are stored in the V-cycle's type, whose values they
+// are, and the V-cycle's last sweep reads its right-hand side in that type.
+// 80 bytes a row and iteration less with FP32 values; a step of the 4.26M beach
+// 158.8 -> 152.8 ms, of the 1.06M tank 11.7 -> 11.2, the same bits.
 // ---------------------------------------------------------------------------
 template <class TI, class TV>
 __device__ __forceinline__ double mg_spmv(int i, int c, double si, const TI* __restrict__ nbr,
                                           const TV* __restrict__ val, size_t ld,
-                                          const double* __restrict__ x) {
-    const double xi = x[i];
+                                          const TV* __restrict__ x) {
+    const double xi = (double)x[i];
     double acc = 0.0;
     int k = 0;
     // loads of four entries ahead of their gathers, sum in entry order
@@ -1047,7 +1060,8 @@ __device__ __forceinline__ double mg_spmv(int i, int c, double si, const TI* __r
         const int j2 = mg_col(nbr[o + 2 * ld], i), j3 = mg_col(nbr[o + 3 * ld], i);
         const double v0 = (double)val[o], v1 = (double)val[o + ld];
         const double v2 = (double)val[o + 2 * ld], v3 = (double)val[o + 3 * ld];
-        const double x0 = x[j0], x1 = x[j1], x2 = x[j2], x3 = x[j3];
+        const double x0 = (double)x[j0], x1 = (double)x[j1];
+        const double x2 = (double)x[j2], x3 = (double)x[j3];
         acc = acc + v0 * (x0 - xi);
         acc = acc + v1 * (x1 - xi);
         acc = acc + v2 * (x2 - xi);
@@ -1055,21 +1069,20 @@ __device__ __forceinline__ double mg_spmv(int i, int c, double si, const TI* __r
     }
     for (; k < c; ++k) {
         const size_t o = (size_t)k * ld + i;
-        acc = acc + (double)val[o] * (x[mg_col(nbr[o], i)] - xi);
+        acc = acc + (double)val[o] * ((double)x[mg_col(nbr[o], i)] - xi);
     }
     return si * xi + acc;
 }
 
-// v = A p^; rv = (r, v); partial (v, rhat)
+// v = A p^; partial (v, rhat)
 template <class TI, class TV>
 __global__ void __launch_bounds__(BLOCK) k_mg_v(int n, size_t ld, const TI* __restrict__ nbr,
                                                 const int* __restrict__ cnt,
                                                 const TV* __restrict__ val,
                                                 const double* __restrict__ rsum,
-                                                const double* __restrict__ ph,
-                                                const double2* __restrict__ rq,
+                                                const TV* __restrict__ ph,
                                                 const double* __restrict__ rhat,
-                                                double2* __restrict__ rv, double* __restrict__ part,
+                                                double* __restrict__ vout, double* __restrict__ part,
                                                 const SolverScalars* sc) {
     // the row's count and row sum are requested before the done test waits
     const int done = sc->done;
@@ -1085,7 +1098,7 @@ __global__ void __launch_bounds__(BLOCK) k_mg_v(int n, size_t ld, const TI* __re
     double v = 0.0;
     if (i < n) {
         const double s = mg_spmv<TI, TV>(i, ci, si, nbr, val, ld, ph);
-        rv[i] = make_double2(rq[i].x, s);
+        vout[i] = s;
         v = s * rhat[i];
     }
     v = block_sum(v);
@@ -1098,7 +1111,7 @@ __global__ void __launch_bounds__(BLOCK) k_mg_t(int n, size_t ld, const TI* __re
                                                 const int* __restrict__ cnt,
                                                 const TV* __restrict__ val,
                                                 const double* __restrict__ rsum,
-                                                const double* __restrict__ sh,
+                                                const TV* __restrict__ sh,
                                                 const double* __restrict__ s,
                                                 double* __restrict__ t, double* __restrict__ part,
                                                 const SolverScalars* sc) {
@@ -1130,15 +1143,14 @@ __global__ void __launch_bounds__(BLOCK) k_mg_t(int n, size_t ld, const TI* __re
     }
 }
 
-// xs += alpha p^ + omega s^; r = s - omega t; q = p - omega v; partials (r, rhat), (r, r)
-__global__ void __launch_bounds__(BLOCK) k_mg_x(int n, const double* __restrict__ p,
-                                                const double* __restrict__ ph,
+// xs += alpha p^ + omega s^; r = s - omega t; partials (r, rhat), (r, r)
+template <class T>
+__global__ void __launch_bounds__(BLOCK) k_mg_x(int n, const T* __restrict__ ph,
                                                 const double* __restrict__ s,
-                                                const double* __restrict__ sh,
+                                                const T* __restrict__ sh,
                                                 const double* __restrict__ t,
-                                                const double2* __restrict__ rv,
                                                 const double* __restrict__ rhat,
-                                                double* __restrict__ xs, double2* __restrict__ rq,
+                                                double* __restrict__ xs, double* __restrict__ r,
                                                 double* __restrict__ part, const SolverScalars* sc) {
     // the scalars and the row's first operands are requested before the
     // done test waits
@@ -1149,17 +1161,16 @@ __global__ void __launch_bounds__(BLOCK) k_mg_x(int n, const double* __restrict_
     double xi = 0.0, phi = 0.0;
     if (i < n) {
         xi = xs[i];
-        phi = ph[i];
+        phi = (double)ph[i];
     }
     if (done) return;
     double v0 = 0.0, v1 = 0.0;
     if (i < n) {
-        xs[i] = (xi + al * phi) + w * sh[i];
-        const double r = s[i] - w * t[i];
-        const double q = p[i] - w * rv[i].y;
-        rq[i] = make_double2(r, q);
-        v0 = r * rhat[i];
-        v1 = r * r;
+        xs[i] = (xi + al * phi) + w * (double)sh[i];
+        const double ri = s[i] - w * t[i];
+        r[i] = ri;
+        v0 = ri * rhat[i];
+        v1 = ri * ri;
     }
     v0 = block_sum(v0);
     v1 = block_sum(v1);
@@ -1167,6 +1178,28 @@ __global__ void __launch_bounds__(BLOCK) k_mg_x(int n, const double* __restrict_
         part[lb] = v0;
         part[gridDim.x + lb] = v1;
     }
+}
+
+// START: rhat = r, xs = 0, partial (r, r): a first iteration or a restart.
+// Otherwise partial (r, rhat): r replaced by the true residual.
+template <bool START>
+__global__ void __launch_bounds__(BLOCK) k_mg_start(int n, const double* __restrict__ r,
+                                                    double* __restrict__ rhat,
+                                                    double* __restrict__ xs,
+                                                    double* __restrict__ part) {
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int i = lb * BLOCK + threadIdx.x;
+    double v = 0.0;
+    if (i < n) {
+        const double ri = r[i];
+        if (START) {
+            rhat[i] = ri;
+            xs[i] = 0.0;
+        }
+        v = ri * (START ? ri : rhat[i]);
+    }
+    v = block_sum(v);
+    if (threadIdx.x == 0) part[lb] = v;
 }
 
 // FP32 values and FP64 row sums of a Jacobi-scaled FP64 matrix in the
@@ -1379,17 +1412,16 @@ static int mg_join(isph_ctx* c) {
     return ISPH_OK;
 }
 
-// one V-cycle: b formed from `pairs` (MODE 0: p from rq, MODE 1: s from rv)
-// into bout, preconditioned vector into out
-template <class T, class TI, int MODE, bool FIRST>
-static void mg_vcycle(isph_ctx* c, const MGSystem& sys, const TI* nbr, const double2* pairs,
-                      double* bout, double* out) {
+// one V-cycle: b formed into bout (MODE 0: p, MODE 1: s), preconditioned
+// vector into out
+template <class T, int MODE, bool FIRST>
+static void mg_vcycle(isph_ctx* c, double* bout, T* out) {
     MGData* m = c->mg;
     const GridInfo& g = c->grid;
     const int n = c->n;
     const size_t ld = (size_t)c->cap;
-    k_mg_bpoint<T, MODE, FIRST><<<nblk(n), BLOCK, 0, c->stream>>>(n, pairs, c->sc, bout,
-                                                                   as<T>(m->z0));
+    k_mg_bpoint<T, MODE, FIRST><<<nblk(n), BLOCK, 0, c->stream>>>(
+        n, c->v64[9], c->v64[7], c->sc, bout, as<T>(m->z0));
     k_mg_restrict1<T><<<nblk((int64_t)g.nx * g.ny), BLOCK, 0, c->stream>>>(
         g, c->bincnt, as<T>(m->z0), as<T>(m->lv[0].b), c->sc);
     const int lb = m->lb;
@@ -1429,8 +1461,9 @@ static void mg_vcycle(isph_ctx* c, const MGSystem& sys, const TI* nbr, const dou
         std::swap(b.x, b.x2);
         std::swap(a.x, a.x2);
     }
-    k_mg_fine_up<T><<<nblk(n), BLOCK, 0, c->stream>>>(n, ld, g.ny, m->cell, mg_p9<T>(m), bout,
-                                                       as<T>(m->lv[0].x), MG_OVER, out, c->sc);
+    k_mg_fine_up<T><<<nblk(n), BLOCK, 0, c->stream>>>(n, ld, g.ny, m->cell, mg_p9<T>(m),
+                                                       as<T>(m->z0), as<T>(m->lv[0].x), MG_OVER,
+                                                       out, c->sc);
 }
 
 template <class T, class TI>
@@ -1441,7 +1474,8 @@ static int mg_iterate(isph_ctx* c, const MGSystem& sys, const TI* nbr, const Sol
     const int n = c->n;
     const size_t ld = (size_t)c->cap;
     double *rhat = c->v64[0], *p = c->v64[1], *s = c->v64[2], *t = c->v64[3], *xs = c->v64[4];
-    double *ph = c->v64[5], *sh = c->v64[6];
+    T *ph = as<T>(c->v64[5]), *sh = as<T>(c->v64[6]);
+    double *v = c->v64[7], *r = c->v64[9];
     if (int rc = mg_join(c)) return rc;
     for (;;) {
         int batch = 4;
@@ -1453,18 +1487,17 @@ static int mg_iterate(isph_ctx* c, const MGSystem& sys, const TI* nbr, const Sol
         }
         for (int b = 0; b < batch; ++b) {
             if (first)
-                mg_vcycle<T, TI, 0, true>(c, sys, nbr, c->rq64, p, ph);
+                mg_vcycle<T, 0, true>(c, p, ph);
             else
-                mg_vcycle<T, TI, 0, false>(c, sys, nbr, c->rq64, p, ph);
+                mg_vcycle<T, 0, false>(c, p, ph);
             k_mg_v<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, ph,
-                                                          c->rq64, rhat, c->rv64, c->part, c->sc);
+                                                          rhat, v, c->part, c->sc);
             k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_ALPHA, grid, c->part, c->sc, ctl);
-            mg_vcycle<T, TI, 1, false>(c, sys, nbr, c->rv64, s, sh);
+            mg_vcycle<T, 1, false>(c, s, sh);
             k_mg_t<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, sh, s,
                                                           t, c->part, c->sc);
             k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_OMEGA, grid, c->part, c->sc, ctl);
-            k_mg_x<<<grid, BLOCK, 0, c->stream>>>(n, p, ph, s, sh, t, c->rv64, rhat, xs, c->rq64,
-                                                   c->part, c->sc);
+            k_mg_x<T><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, c->part, c->sc);
             k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, c->part, c->sc, ctl);
             first = false;
         }
@@ -1479,7 +1512,7 @@ template <class T, class TI>
 static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
     const int grid = nblk8(c->n);
     double* x = sys.x;
-    double* r64 = c->v64[9];
+    double* r64 = c->v64[9];  // the true residual, replaced by the recurrence's
     int rc = mg_setup<T, TI>(c, sys, nbr);
     if (rc) return rc;
     SolveCtl ctl = solve_ctl(c, 1);
@@ -1496,8 +1529,7 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
         return ISPH_OK;
     }
     if (c->sc_host->done == DONE_CONVERGED) return ISPH_OK;
-    k_mx_start<double><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->rq64, c->v64[0], c->v64[4],
-                                                      c->part, c->sc);
+    k_mg_start<true><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4], c->part);
     k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, ctl);
     HIPCHK(c, hipGetLastError());
     if ((rc = read_sc(c))) return rc;
@@ -1516,13 +1548,13 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
         if (c->sc_host->done == DONE_FAILED)
             return fail(c, ISPH_E_NOCONV, "multigrid PPE solve did not converge");
         if (c->sc_host->brk) {
-            k_mx_start<double><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->rq64, c->v64[0],
-                                                              c->v64[4], c->part, c->sc);
+            k_mg_start<true><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4],
+                                                            c->part);
             k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, ctl);
             first = true;
         } else {
-            k_mx_replace<double><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->rq64, c->v64[0],
-                                                                c->part, c->sc);
+            k_mg_start<false><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4],
+                                                             c->part);
             k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_REPLACE, grid, c->part, c->sc, ctl);
         }
         HIPCHK(c, hipGetLastError());
