@@ -103,11 +103,11 @@ int alloc_ckpt(isph_ctx* c, Ckpt& k) {
 int save_ckpt(isph_ctx* c, Ckpt& k) {
     int rc = alloc_ckpt(c, k);
     if (rc) return fail(c, ISPH_E_HIP, "adjoint checkpoint allocation failed");
-    if ((rc = copy_state(c, c->st[c->cur], k.v, c->n))) return rc;
-    HIPCHK(c, hipMemcpyAsync(k.key, c->key_s, sizeof(int) * c->n, hipMemcpyDeviceToDevice,
-                             c->stream));
-    HIPCHK(c, hipMemcpyAsync(k.bins, c->bincnt, sizeof(int) * (c->grid.nbins + 2),
-                             hipMemcpyDeviceToDevice, c->stream));
+    ArrayCopy l[STATE_ARRAYS + 2];
+    int m = state_copies(c->st[c->cur], k.v, c->n, l);
+    l[m++] = ArrayCopy{c->key_s, k.key, sizeof(int) * c->n};
+    l[m++] = ArrayCopy{c->bincnt, k.bins, sizeof(int) * (c->grid.nbins + 2)};
+    if ((rc = copy_arrays(c, l, m))) return rc;
     HIPCHK(c, hipMemcpyAsync(&k.ss, c->ss, sizeof(SimScalars), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     k.n = c->n;
@@ -115,12 +115,12 @@ int save_ckpt(isph_ctx* c, Ckpt& k) {
 }
 
 int load_ckpt(isph_ctx* c, const Ckpt& k) {
-    int rc = copy_state(c, k.v, c->st[c->cur], k.n);
+    ArrayCopy l[STATE_ARRAYS + 2];
+    int m = state_copies(k.v, c->st[c->cur], k.n, l);
+    l[m++] = ArrayCopy{k.key, c->key_s, sizeof(int) * k.n};
+    l[m++] = ArrayCopy{k.bins, c->bincnt, sizeof(int) * (c->grid.nbins + 2)};
+    int rc = copy_arrays(c, l, m);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->key_s, k.key, sizeof(int) * k.n, hipMemcpyDeviceToDevice,
-                             c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->bincnt, k.bins, sizeof(int) * (c->grid.nbins + 2),
-                             hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->ss, &k.ss, sizeof(SimScalars), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->n = k.n;
@@ -289,50 +289,51 @@ int dsum(isph_ctx* c, int64_t count, const double* x, double* out) {
     return ISPH_OK;
 }
 
-int copy_dev(isph_ctx* c, void* dst, const void* src, size_t bytes) {
-    HIPCHK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, c->stream));
-    return ISPH_OK;
+// what the tape keeps of a re-binning and the search after it
+int tape_search(isph_ctx* c, int* perm, double* rho, int* nbr, int* cnt, double* L) {
+    const size_t N = (size_t)c->cap, M = (size_t)c->prm.max_nbr, n = (size_t)c->n;
+    const ArrayCopy l[] = {{c->perm, perm, sizeof(int) * n},
+                           {c->st[c->cur].rho, rho, sizeof(double) * n},
+                           {c->nbr, nbr, sizeof(int) * N * M},
+                           {c->cnt, cnt, sizeof(int) * n},
+                           {c->L, L, sizeof(double) * 4 * n}};
+    return copy_arrays(c, l, 5);
 }
 
 // one step of main.f90:41-66 (the run_step order) recording the tape
 int tape_step(isph_ctx* c, StepTape& t) {
-    const size_t N = (size_t)c->cap, M = (size_t)c->prm.max_nbr;
     int rc;
     if ((rc = copy_state(c, c->st[c->cur], t.Sa, c->n))) return rc;
     k_advance_time<<<1, 64, 0, c->stream>>>(c->ss);
     if ((rc = run_projection(c))) return rc;
     if ((rc = sort_particles(c, false, false))) return rc;
-    if ((rc = copy_dev(c, t.perm1, c->perm, sizeof(int) * c->n))) return rc;
-    if ((rc = copy_dev(c, t.rho0, c->st[c->cur].rho, sizeof(double) * c->n))) return rc;
     if ((rc = run_neighbour(c))) return rc;
-    if ((rc = copy_dev(c, t.nbr1, c->nbr, sizeof(int) * N * M))) return rc;
-    if ((rc = copy_dev(c, t.cnt1, c->cnt, sizeof(int) * c->n))) return rc;
-    if ((rc = copy_dev(c, t.L1, c->L, sizeof(double) * 4 * c->n))) return rc;
+    if ((rc = tape_search(c, t.perm1, t.rho0, t.nbr1, t.cnt1, t.L1))) return rc;
     if ((rc = run_effpor(c))) return rc;
     if ((rc = run_eddyvis(c))) return rc;
     if ((rc = run_int_vel(c))) return rc;
     if ((rc = run_assemble(c))) return rc;
-    if ((rc = copy_state(c, c->st[c->cur], t.Sc, c->n))) return rc;
-    if ((rc = copy_dev(c, t.ssc, c->ss, sizeof(SimScalars)))) return rc;
+    ArrayCopy l[STATE_ARRAYS + 1];
+    int k = state_copies(c->st[c->cur], t.Sc, c->n, l);
+    l[k++] = ArrayCopy{c->ss, t.ssc, sizeof(SimScalars)};
+    if ((rc = copy_arrays(c, l, k))) return rc;
     if ((rc = run_solve(c))) return rc;
     if ((rc = take_errors(c))) return rc;
-    if ((rc = copy_dev(c, t.p, c->st[c->cur].p, sizeof(double) * c->n))) return rc;
     if ((rc = run_comp_vel(c))) return rc;
-    if ((rc = copy_dev(c, t.vel1, c->st[c->cur].vel, sizeof(double2) * c->n))) return rc;
+    const ArrayCopy l2[] = {{c->st[c->cur].p, t.p, sizeof(double) * c->n},
+                            {c->st[c->cur].vel, t.vel1, sizeof(double2) * c->n}};
+    if ((rc = copy_arrays(c, l2, 2))) return rc;
     if ((rc = run_comp_pos(c))) return rc;
     if ((rc = sort_particles(c, true, false))) return rc;
-    if ((rc = copy_dev(c, t.perm2, c->perm, sizeof(int) * c->n))) return rc;
-    if ((rc = copy_dev(c, t.rho1p, c->st[c->cur].rho, sizeof(double) * c->n))) return rc;
     if ((rc = run_neighbour(c))) return rc;
-    if ((rc = copy_dev(c, t.nbr2, c->nbr, sizeof(int) * N * M))) return rc;
-    if ((rc = copy_dev(c, t.cnt2, c->cnt, sizeof(int) * c->n))) return rc;
-    if ((rc = copy_dev(c, t.L2, c->L, sizeof(double) * 4 * c->n))) return rc;
+    if ((rc = tape_search(c, t.perm2, t.rho1p, t.nbr2, t.cnt2, t.L2))) return rc;
     if ((rc = run_freesurf(c))) return rc;
     if ((rc = run_effpor(c))) return rc;
     if ((rc = copy_state(c, c->st[c->cur], t.Sf, c->n))) return rc;
     if ((rc = run_shift(c))) return rc;
     if ((rc = run_timestep(c))) return rc;
-    if ((rc = copy_dev(c, t.ssend, c->ss, sizeof(SimScalars)))) return rc;
+    const ArrayCopy l3[] = {{c->ss, t.ssend, sizeof(SimScalars)}};
+    if ((rc = copy_arrays(c, l3, 1))) return rc;
     return sync_check(c);
 }
 

@@ -213,18 +213,15 @@ int run_projection(isph_ctx* c) {
 
 int run_neighbour(isph_ctx* c) {
     const isph_params& p = c->prm;
-    if (c->n)
-        k_neighbour<<<nblk(c->n), BLOCK, 0, c->stream>>>(
-            c->n, c->grid, kconsts(c), p.lamfs * p.maxdivr, p.max_nbr, (size_t)c->cap,
-            c->st[c->cur], c->key_s, c->bincnt, c->nbr, c->cnt, c->L, c->divr, c->err);
-    HIPCHK(c, hipGetLastError());
     // the lists keep these positions' distances (the reference stores dist and
     // klt per pair, search.f90:65-74): the stages of the salt-water step that
     // run after the shift has moved the particles (scalart, the last eddyvis)
-    // take their pair distances from here
+    // take their pair distances from pos_nb
     if (c->n)
-        HIPCHK(c, hipMemcpyAsync(c->pos_nb, c->st[c->cur].pos, sizeof(double2) * c->n,
-                                 hipMemcpyDeviceToDevice, c->stream));
+        k_neighbour<<<nblk(c->n), BLOCK, 0, c->stream>>>(
+            c->n, c->grid, kconsts(c), p.lamfs * p.maxdivr, p.max_nbr, (size_t)c->cap,
+            c->st[c->cur], c->key_s, c->bincnt, c->nbr, c->cnt, c->L, c->divr, c->pos_nb, c->err);
+    HIPCHK(c, hipGetLastError());
     c->have_nbr = true;
     c->assembled = false;
     return ISPH_OK;
@@ -726,21 +723,27 @@ int run_step(isph_ctx* c) {
     return ISPH_OK;
 }
 
-int copy_state(isph_ctx* c, const StateView& a, const StateView& b, int n) {
-    auto D2D = hipMemcpyDeviceToDevice;
+int state_copies(const StateView& a, const StateView& b, int n, ArrayCopy* out) {
     const size_t n2 = sizeof(double2) * n, nd = sizeof(double) * n, ni = sizeof(int) * n;
-    HIPCHK(c, hipMemcpyAsync(b.pos, a.pos, n2, D2D, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b.vel, a.vel, n2, D2D, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b.sp, a.sp, n2, D2D, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b.sv, a.sv, n2, D2D, c->stream));
+    int k = 0;
+    auto add = [&](void* dst, const void* src, size_t bytes) { out[k++] = ArrayCopy{src, dst, bytes}; };
+    add(b.pos, a.pos, n2);
+    add(b.vel, a.vel, n2);
+    add(b.sp, a.sp, n2);
+    add(b.sv, a.sv, n2);
     const double* da[] = {a.mass, a.rho, a.oden, a.p,     a.por, a.R,
                           a.nut,  a.tke, a.varts, a.velm, a.con, a.ovol};
     double* db[] = {b.mass, b.rho, b.oden, b.p, b.por, b.R, b.nut, b.tke, b.varts, b.velm, b.con, b.ovol};
-    for (int k = 0; k < 12; ++k) HIPCHK(c, hipMemcpyAsync(db[k], da[k], nd, D2D, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b.tid, a.tid, ni, D2D, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b.flags, a.flags, ni, D2D, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b.pid, a.pid, ni, D2D, c->stream));
-    return ISPH_OK;
+    for (int j = 0; j < 12; ++j) add(db[j], da[j], nd);
+    add(b.tid, a.tid, ni);
+    add(b.flags, a.flags, ni);
+    add(b.pid, a.pid, ni);
+    return k;
+}
+
+int copy_state(isph_ctx* c, const StateView& a, const StateView& b, int n) {
+    ArrayCopy l[STATE_ARRAYS];
+    return copy_arrays(c, l, state_copies(a, b, n, l));
 }
 
 }  // namespace host
@@ -1273,13 +1276,13 @@ int isph_checkpoint(isph_ctx* c, int32_t slot) {
             return fail(c, ISPH_E_HIP, "checkpoint allocation failed");
         }
     }
-    int rc = copy_state(c, c->st[c->cur], sl.v, c->n);
+    ArrayCopy l[STATE_ARRAYS + 3];
+    int k = state_copies(c->st[c->cur], sl.v, c->n, l);
+    l[k++] = ArrayCopy{c->key_s, sl.key, sizeof(int) * c->n};
+    l[k++] = ArrayCopy{c->fsol, sl.fsol, sizeof(double) * c->cap};
+    l[k++] = ArrayCopy{c->bincnt, sl.bins, sizeof(int) * (c->grid.nbins + 2)};
+    int rc = copy_arrays(c, l, k);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(sl.key, c->key_s, sizeof(int) * c->n, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(sl.fsol, c->fsol, sizeof(double) * c->cap, hipMemcpyDeviceToDevice,
-                             c->stream));
-    HIPCHK(c, hipMemcpyAsync(sl.bins, c->bincnt, sizeof(int) * (c->grid.nbins + 2),
-                             hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(&sl.ss, c->ss, sizeof(SimScalars), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     sl.n = c->n;
@@ -1297,13 +1300,13 @@ int isph_restore(isph_ctx* c, int32_t slot) {
     if (!sl.used) return fail(c, ISPH_E_STATE, "restore from an empty checkpoint slot");
     if (sl.nzones != c->nzones)
         return fail(c, ISPH_E_STATE, "buffer zones were installed or removed since this checkpoint");
-    int rc = copy_state(c, sl.v, c->st[c->cur], sl.n);
+    ArrayCopy l[STATE_ARRAYS + 3];
+    int k = state_copies(sl.v, c->st[c->cur], sl.n, l);
+    l[k++] = ArrayCopy{sl.key, c->key_s, sizeof(int) * sl.n};
+    l[k++] = ArrayCopy{sl.fsol, c->fsol, sizeof(double) * c->cap};
+    l[k++] = ArrayCopy{sl.bins, c->bincnt, sizeof(int) * (c->grid.nbins + 2)};
+    int rc = copy_arrays(c, l, k);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->key_s, sl.key, sizeof(int) * sl.n, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->fsol, sl.fsol, sizeof(double) * c->cap, hipMemcpyDeviceToDevice,
-                             c->stream));
-    HIPCHK(c, hipMemcpyAsync(c->bincnt, sl.bins, sizeof(int) * (c->grid.nbins + 2),
-                             hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->ss, &sl.ss, sizeof(SimScalars), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->n = sl.n;

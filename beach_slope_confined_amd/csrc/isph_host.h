@@ -177,6 +177,18 @@ int download(isph_ctx* c, int64_t rows, const Column* cols, int ncol);
 void transfer_attach();  // a context lives: the staging memory is kept
 void transfer_detach();
 
+// device arrays that do not overlap, copied in stream order by one launch for
+// up to 24 of them (isph_copy.hip); bytes a multiple of 4
+struct ArrayCopy {
+    const void* src;
+    void* dst;
+    size_t bytes;
+};
+int copy_arrays(isph_ctx* c, const ArrayCopy* a, int n);
+constexpr int STATE_ARRAYS = 19;
+// the copies of the first n rows of state a to b; returns STATE_ARRAYS
+int state_copies(const StateView& a, const StateView& b, int n, ArrayCopy* out);
+
 int alloc_state(isph_ctx* c, StateView& s, size_t cap);
 void free_state(StateView& s);
 int copy_state(isph_ctx* c, const StateView& a, const StateView& b, int n);

@@ -339,7 +339,7 @@ __global__ void k_gather_state(int n, const int* perm, StateView src, StateView 
 __global__ void k_projection(int n, StateView s, const SimScalars* ss);
 __global__ void k_neighbour(int n, GridInfo g, KernelConsts kc, double thr, int maxnbr, size_t ld,
                             StateView s, const int* key, const int* bstart, int* nbr, int* cnt,
-                            double* L, double* divr, uint32_t* err);
+                            double* L, double* divr, double2* pos_nb, uint32_t* err);
 __global__ void k_effpor(int n, GridInfo g, KernelConsts kc, PorousParams pp, StateView s,
                          const int* key, const double2* spos, const double* sm, const double* sr,
                          const int* sstart, uint32_t* err);

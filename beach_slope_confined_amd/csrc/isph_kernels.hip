@@ -284,7 +284,8 @@ __global__ void __launch_bounds__(BLOCK) k_neighbour(int n, GridInfo g, KernelCo
                                                      const int* __restrict__ bstart,
                                                      int* __restrict__ nbr, int* __restrict__ cnt,
                                                      double* __restrict__ L,
-                                                     double* __restrict__ divr, uint32_t* err) {
+                                                     double* __restrict__ divr,
+                                                     double2* __restrict__ pos_nb, uint32_t* err) {
     // the first NB_STAGE entries of each list are kept in LDS and stored after
     // the scan, slot by slot, so that a wave's stores of slot k are one
     // coalesced row segment (stored as found, the lanes' k-th entries arrive
@@ -313,6 +314,7 @@ __global__ void __launch_bounds__(BLOCK) k_neighbour(int n, GridInfo g, KernelCo
     if (i >= n) return;
     const int R = key[i] / g.per;
     const double2 pi = s.pos[i];
+    pos_nb[i] = pi;
     const double t2 = (kc.twoh * kc.twoh) * (1.0 + 0x1p-30);
     int lo[3], hi[3];
     for (int w = 0; w < 3; ++w) {
