@@ -494,13 +494,13 @@ int iterate(isph_ctx* c, const KrylovArgs<TV, TX, TI>& a, const SolveCtl& ctl, b
             else
                 k_krylov_1t<TV, TX, TI, false><<<grid, BLOCK, 0, c->stream>>>(a, c->sc);
             prof_record(c, k0, false);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_ALPHA, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_ALPHA, grid, c->part, c->sc, c->sc, ctl);
             prof_record(c, k0 + 1, true);
             k_krylov_2<TV, TX, TI><<<grid, BLOCK, 0, c->stream>>>(a, c->sc);
             prof_record(c, k0 + 1, false);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_OMEGA, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_OMEGA, grid, c->part, c->sc, c->sc, ctl);
             k_krylov_3<TV, TX, TI><<<grid, BLOCK, 0, c->stream>>>(a, c->sc);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, c->part, c->sc, c->sc, ctl);
             first = false;
         }
         HIPCHK(c, hipGetLastError());
@@ -522,7 +522,7 @@ int solve_fp64_t(isph_ctx* c, const TI* nbr, const double* val, const double* rh
     ResidArgs ra = resid_args(c, x, c->v64[9], val, rhs);
     if constexpr (std::is_same<TI, short>::value) ra.nbr16 = nbr;
     k_resid<<<grid, BLOCK, 0, c->stream>>>(ra, 1, c->rq64, c->v64[0]);
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_INIT, grid, c->part, c->sc, ctl);
+    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_INIT, grid, c->part, c->sc, c->sc, ctl);
     HIPCHK(c, hipGetLastError());
     int rc = read_sc(c);
     if (rc) return rc;
@@ -537,7 +537,7 @@ int solve_fp64_t(isph_ctx* c, const TI* nbr, const double* val, const double* rh
         if (d == DONE_FAILED) return fail(c, ISPH_E_NOCONV, "PPE solve did not converge");
         if (d == DONE_RECURRENCE) {
             k_resid<<<grid, BLOCK, 0, c->stream>>>(ra, 1, c->rq64, c->v64[0]);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_TRUE, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_TRUE, grid, c->part, c->sc, c->sc, ctl);
             HIPCHK(c, hipGetLastError());
             if ((rc = read_sc(c))) return rc;
             first = true;
@@ -579,8 +579,8 @@ int solve_mixed_t(isph_ctx* c, const TI* nbr, TX* const* v, typename Pair2<TX>::
     ResidArgs ra = resid_args(c, x, r64);
     if constexpr (std::is_same<TI, short>::value) ra.nbr16 = nbr;
     k_resid<<<grid, BLOCK, 0, c->stream>>>(ra, 0, nullptr, nullptr);
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_INIT, grid, c->part, c->sc, solve_ctl(c, 0));
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, ctl);
+    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_INIT, grid, c->part, c->sc, c->sc, solve_ctl(c, 0));
+    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, c->sc, ctl);
     HIPCHK(c, hipGetLastError());
     int rc = read_sc(c);
     if (rc) return rc;
@@ -590,7 +590,7 @@ int solve_mixed_t(isph_ctx* c, const TI* nbr, TX* const* v, typename Pair2<TX>::
     }
     if (c->sc_host->done == DONE_CONVERGED) return ISPH_OK;
     k_mx_start<TX><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, rq, v[0], v[4], c->part, c->sc);
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, ctl);
+    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, c->sc, ctl);
     HIPCHK(c, hipGetLastError());
     if ((rc = read_sc(c))) return rc;
     bool first = true;
@@ -602,7 +602,7 @@ int solve_mixed_t(isph_ctx* c, const TI* nbr, TX* const* v, typename Pair2<TX>::
         // reliable update: flush x, FP64 true residual, replace r
         k_mx_flush<TX><<<nblk(c->n), BLOCK, 0, c->stream>>>(c->n, x, v[4]);
         k_resid<<<grid, BLOCK, 0, c->stream>>>(ra, 0, nullptr, nullptr);
-        k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, ctl_flush);
+        k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, c->sc, ctl_flush);
         HIPCHK(c, hipGetLastError());
         if ((rc = read_sc(c))) return rc;
         if (c->sc_host->done == DONE_CONVERGED) return ISPH_OK;
@@ -612,11 +612,11 @@ int solve_mixed_t(isph_ctx* c, const TI* nbr, TX* const* v, typename Pair2<TX>::
             // breakdown, or iterative refinement: the next correction starts
             // from zero on the true residual, rhat = r
             k_mx_start<TX><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, rq, v[0], v[4], c->part, c->sc);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, c->sc, ctl);
             first = true;
         } else {
             k_mx_replace<TX><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, rq, v[0], c->part, c->sc);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_REPLACE, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_REPLACE, grid, c->part, c->sc, c->sc, ctl);
         }
         HIPCHK(c, hipGetLastError());
     }
@@ -822,7 +822,7 @@ int isph_create(const isph_params* prm, int32_t cap, int32_t cap_soil, isph_ctx*
     rc |= dalloc(c, &c->part, 4 * (size_t)nblk8(cap));
     rc |= dalloc(c, &c->counters, 16);
     rc |= dalloc(c, &c->gs_words, (size_t)gs_words(GS_PARTS));
-    rc |= dalloc(c, &c->sc, 1);
+    rc |= dalloc(c, &c->sc, 2);
     rc |= dalloc(c, &c->ss, 1);
     rc |= dalloc(c, &c->err, 2);
     rc |= dalloc(c, &c->spos, (size_t)std::max(cap_soil, 1));

@@ -360,7 +360,8 @@ template <class TV, class TX, class TI>
 __global__ void k_krylov_2(KrylovArgs<TV, TX, TI> a, const SolverScalars* sc);
 template <class TV, class TX, class TI>
 __global__ void k_krylov_3(KrylovArgs<TV, TX, TI> a, const SolverScalars* sc);
-__global__ void k_finish(int kind, int nbp, const double* part, SolverScalars* sc, SolveCtl ctl);
+__global__ void k_finish(int kind, int nbp, const double* part, const SolverScalars* sc,
+                         SolverScalars* out, SolveCtl ctl);
 __global__ void k_resid(ResidArgs a, int mode, double2* rq, double* rhat);
 template <class TX>
 __global__ void k_mx_start(int n, const double* r64, typename Pair2<TX>::type* rq, TX* rhat,

@@ -46,6 +46,7 @@
 #include <vector>
 
 #include "isph_host.h"
+#include "isph_finish.h"
 #include "isph_kernels.h"
 
 namespace isph {
@@ -196,6 +197,70 @@ __global__ void k_mg_galerkin(int nx, int ny, const T* __restrict__ A, int nx2, 
 // ---------------------------------------------------------------------------
 // V-cycle kernels (value type T: float for MIXED_MG, double for FP64_MG)
 // ---------------------------------------------------------------------------
+// A reduction finished by the kernels that use its result: every block sums the
+// partials itself, in k_finish's tree (256 threads stand for its 1024), and forms
+// the same scalars; block 0 stores them for the kernels after.  `in` and `out`
+// differ, as other blocks may still be reading `in`.  A launch of one block
+// (3.4 us on the stream, three of an iteration's 20) becomes a few loads and a
+// wave's sums in each block.  Up to one partial for each thread of k_finish,
+// 262k rows, where it still wins: three steps at 1.3k rows 6.38 -> 5.89 ms, 55k
+// 12.37 -> 11.89, one at 164k 3.61 -> 3.47, 255k 3.83 -> 3.77; beyond, a block
+// would sum more partials than it has rows to work on.
+struct MGFin {
+    int kind, nbp;
+    const double* part;
+    const SolverScalars* in;
+    SolverScalars* out;
+    SolveCtl ctl;
+};
+constexpr int MG_FIN_MAX = FIN_BLOCK;  // partials: one a thread of k_finish
+
+template <bool FIN>
+__device__ __forceinline__ SolverScalars mg_scalars(const MGFin& f) {
+    if (!FIN) return *f.in;
+    __shared__ double red[2][FIN_BLOCK / 64];
+    constexpr int Q = FIN_BLOCK / BLOCK;
+    const bool two = f.kind != FIN_ALPHA;
+    const int t = threadIdx.x;
+    double p0[Q], p1[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int k = q * BLOCK + t;
+        p0[q] = k < f.nbp ? f.part[k] : 0.0;
+        p1[q] = two && k < f.nbp ? f.part[f.nbp + k] : 0.0;
+    }
+    SolverScalars s = *f.in;
+    if (!s.done) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int w = q * (BLOCK / 64) + t / 64;
+            double a = 0.0, b = 0.0;
+            if (w * 64 < f.nbp) {  // a wave of k_finish past the partials sums zeros
+                a = wave_sum(0.0 + p0[q]);
+                if (two) b = wave_sum(0.0 + p1[q]);
+            }
+            if ((t & 63) == 0) {
+                red[0][w] = a;
+                red[1][w] = b;
+            }
+        }
+        __syncthreads();
+        double sum[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            double a[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) a[k] = red[u][2 * k] + red[u][2 * k + 1];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) a[k] = a[2 * k] + a[2 * k + 1];
+            sum[u] = (a[0] + a[1]) + (a[2] + a[3]);
+        }
+        finish_update(f.kind, sum[0], two ? sum[1] : 0.0, s, f.ctl);
+    }
+    if (blockIdx.x == 0 && t == 0) *f.out = s;
+    return s;
+}
+
 // Level 0 down: the V-cycle's right-hand side and its restriction to the cells.
 // MODE 0: b = p = r + beta q, q = p - omega v (p = r on a restart);
 // MODE 1: b = s = r - alpha v.
@@ -209,23 +274,28 @@ __global__ void k_mg_galerkin(int nx, int ny, const T* __restrict__ A, int nx2, 
 // r0 in memory, took 3.4 + 3.7 us at 133k rows and 22 + 12.8 us at 4.26M.
 constexpr int MG_RCELLS = 64;  // cells of a block
 constexpr int MG_RROWS = 1024; // rows of a block kept in LDS (9 to 16 a filled cell)
-template <class T, int MODE, bool FIRST>
+template <class T, int MODE, bool FIRST, bool FIN>
 __global__ void __launch_bounds__(BLOCK) k_mg_down0(GridInfo g, const int* __restrict__ bstart,
                                                     const double* __restrict__ r,
-                                                    const double* __restrict__ v,
-                                                    const SolverScalars* sc,
+                                                    const double* __restrict__ v, MGFin fin,
                                                     double* __restrict__ bout,
                                                     T* __restrict__ r0, T* __restrict__ b1) {
     __shared__ T rs[MG_RROWS];
-    // the flag, the coefficients and the bin starts are requested together
-    const int done = sc->done;
-    const double coef = MODE == 0 ? sc->betas : sc->alpha, w = sc->wi;
+    // the scalars and the bin starts are requested together
     const int nc = g.nx * g.ny, t = threadIdx.x;
     const int k0 = xcd_tile(blockIdx.x, gridDim.x) * MG_RCELLS, k1 = min(k0 + MG_RCELLS, nc);
     const int i0 = bstart[g.per * k0], i1 = bstart[g.per * k1];
     const int k = min(k0 + t, k1 - 1);  // rank of the thread's cell
     const int lo = bstart[g.per * k], hi = bstart[g.per * (k + 1)];
-    if (done) return;
+    const int cx = k / g.ny, cy = k - cx * g.ny;
+    const int cell = g.order ? cx * g.ny + (g.ny - 1 - cy) : k;
+    if (FIN && i0 == i1 && blockIdx.x != 0) {  // no rows: no need of the scalars
+        if (k0 + t < k1) b1[cell] = (T)0;
+        return;
+    }
+    const SolverScalars sc = mg_scalars<FIN>(fin);
+    if (sc.done) return;
+    const double coef = MODE == 0 ? sc.betas : sc.alpha, w = sc.wi;
     for (int i = i0 + t; i < i1; i += BLOCK) {
         const double ri = r[i];
         double bi = ri;
@@ -240,8 +310,7 @@ __global__ void __launch_bounds__(BLOCK) k_mg_down0(GridInfo g, const int* __res
     if (k0 + t >= k1) return;
     T s = (T)0;
     for (int i = lo; i < hi; ++i) s += i - i0 < MG_RROWS ? rs[i - i0] : r0[i];
-    const int cx = k / g.ny, cy = k - cx * g.ny;
-    b1[g.order ? cx * g.ny + (g.ny - 1 - cy) : k] = s;
+    b1[cell] = s;
 }
 
 // neighbour index clamped into [0, n): the stencil entries that point
@@ -1173,18 +1242,16 @@ __global__ void __launch_bounds__(BLOCK) k_mg_t(int n, size_t ld, const TI* __re
 }
 
 // xs += alpha p^ + omega s^; r = s - omega t; partials (r, rhat), (r, r)
-template <class T>
+template <class T, bool FIN>
 __global__ void __launch_bounds__(BLOCK) k_mg_x(int n, const T* __restrict__ ph,
                                                 const double* __restrict__ s,
                                                 const T* __restrict__ sh,
                                                 const double* __restrict__ t,
                                                 const double* __restrict__ rhat,
                                                 double* __restrict__ xs, double* __restrict__ r,
-                                                double* __restrict__ part, const SolverScalars* sc) {
+                                                double* __restrict__ part, MGFin fin) {
     // the scalars and the row's first operands are requested before the
     // done test waits
-    const int done = sc->done;
-    const double al = sc->alpha, w = sc->wi;
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int i = lb * BLOCK + threadIdx.x;
     double xi = 0.0, phi = 0.0;
@@ -1192,7 +1259,9 @@ __global__ void __launch_bounds__(BLOCK) k_mg_x(int n, const T* __restrict__ ph,
         xi = xs[i];
         phi = (double)ph[i];
     }
-    if (done) return;
+    const SolverScalars sc = mg_scalars<FIN>(fin);
+    if (sc.done) return;
+    const double al = sc.alpha, w = sc.wi;
     double v0 = 0.0, v1 = 0.0;
     if (i < n) {
         xs[i] = (xi + al * phi) + w * (double)sh[i];
@@ -1443,15 +1512,16 @@ static int mg_join(isph_ctx* c) {
 
 // one V-cycle: b formed into bout (MODE 0: p, MODE 1: s), preconditioned
 // vector into out
-template <class T, int MODE, bool FIRST>
-static void mg_vcycle(isph_ctx* c, double* bout, T* out) {
+template <class T, int MODE, bool FIRST, bool FIN>
+static void mg_vcycle(isph_ctx* c, const MGFin& fin, double* bout, T* out) {
     MGData* m = c->mg;
     const GridInfo& g = c->grid;
     const int n = c->n;
     const size_t ld = (size_t)c->cap;
     const int nc = g.nx * g.ny;
-    k_mg_down0<T, MODE, FIRST><<<(nc + MG_RCELLS - 1) / MG_RCELLS, BLOCK, 0, c->stream>>>(
-        g, c->bincnt, c->v64[9], c->v64[7], c->sc, bout, as<T>(m->z0), as<T>(m->lv[0].b));
+    k_mg_down0<T, MODE, FIRST, FIN><<<(nc + MG_RCELLS - 1) / MG_RCELLS, BLOCK, 0, c->stream>>>(
+        g, c->bincnt, c->v64[9], c->v64[7], fin, bout, as<T>(m->z0), as<T>(m->lv[0].b));
+    const SolverScalars* sc = FIN ? fin.out : fin.in;
     const int lb = m->lb;
     // the grid levels down, two per launch (k_mg_down2), the last one alone
     // when their number is odd
@@ -1461,22 +1531,22 @@ static void mg_vcycle(isph_ctx* c, double* bout, T* out) {
         const int tiles = ((d.nx + MG_TX - 1) / MG_TX) * ((d.ny + MG_TY - 1) / MG_TY);
         k_mg_down2<T><<<tiles, BLOCK, 0, c->stream>>>(
             a.nx, a.ny, as<T>(a.A), as<T>(a.b), as<T>(a.x), b.nx, b.ny, as<T>(b.A), as<T>(b.b),
-            as<T>(b.x), d.nx, d.ny, as<T>(d.b), c->sc);
+            as<T>(b.x), d.nx, d.ny, as<T>(d.b), sc);
     }
     if (l < lb) {
         MGLevel &a = m->lv[l], &b = m->lv[l + 1];
         k_mg_down<T><<<nblk(4 * (int64_t)b.nx * b.ny), BLOCK, 0, c->stream>>>(
-            a.nx, a.ny, as<T>(a.A), as<T>(a.b), as<T>(a.x), b.nx, b.ny, as<T>(b.b), c->sc);
+            a.nx, a.ny, as<T>(a.A), as<T>(a.b), as<T>(a.x), b.nx, b.ny, as<T>(b.b), sc);
     }
     k_mg_block<T><<<1, MG_CMAX, 0, c->stream>>>(m->blk, as<T>(m->lv[lb].b), as<T>(m->lv[lb].x),
-                                                 as<T>(m->ainv), m->aok, c->sc);
+                                                 as<T>(m->ainv), m->aok, sc);
     // up: the odd level alone first, then pairs (k_mg_up2)
     l = lb - 1;
     if (lb & 1) {
         MGLevel &a = m->lv[l], &b = m->lv[l + 1];
         k_mg_grid_up<T><<<nblk((int64_t)a.nx * a.ny), BLOCK, 0, c->stream>>>(
             a.nx, a.ny, as<T>(a.A), as<T>(a.b), as<T>(a.x), b.ny, as<T>(b.x), MG_OVER, as<T>(a.x2),
-            c->sc);
+            sc);
         std::swap(a.x, a.x2);
         --l;
     }
@@ -1485,13 +1555,13 @@ static void mg_vcycle(isph_ctx* c, double* bout, T* out) {
         const int tiles = ((d.nx + MG_TX - 1) / MG_TX) * ((d.ny + MG_TY - 1) / MG_TY);
         k_mg_up2<T><<<tiles, BLOCK, 0, c->stream>>>(
             a.nx, a.ny, as<T>(a.A), as<T>(a.b), as<T>(a.x), b.nx, b.ny, as<T>(b.A), as<T>(b.b),
-            as<T>(b.x), d.nx, d.ny, as<T>(d.x), MG_OVER, as<T>(b.x2), as<T>(a.x2), c->sc);
+            as<T>(b.x), d.nx, d.ny, as<T>(d.x), MG_OVER, as<T>(b.x2), as<T>(a.x2), sc);
         std::swap(b.x, b.x2);
         std::swap(a.x, a.x2);
     }
     k_mg_fine_up<T><<<nblk(n), BLOCK, 0, c->stream>>>(n, ld, g.ny, m->cell, mg_p9<T>(m),
                                                        as<T>(m->z0), as<T>(m->lv[0].x), MG_OVER,
-                                                       out, c->sc);
+                                                       out, sc);
 }
 
 template <class T, class TI>
@@ -1504,6 +1574,9 @@ static int mg_iterate(isph_ctx* c, const MGSystem& sys, const TI* nbr, const Sol
     double *rhat = c->v64[0], *p = c->v64[1], *s = c->v64[2], *t = c->v64[3], *xs = c->v64[4];
     T *ph = as<T>(c->v64[5]), *sh = as<T>(c->v64[6]);
     double *v = c->v64[7], *r = c->v64[9];
+    // k_mg_x's partials: apart from k_mg_t's, which its other blocks may be reading
+    double* part_x = c->part + 2 * (size_t)grid;
+    const bool own = grid <= MG_FIN_MAX;
     if (int rc = mg_join(c)) return rc;
     for (;;) {
         int batch = 4;
@@ -1513,20 +1586,43 @@ static int mg_iterate(isph_ctx* c, const MGSystem& sys, const TI* nbr, const Sol
             const double ratio = std::sqrt(h.rr) / target;
             batch = ratio > 100.0 ? 8 : (ratio > 3.0 ? 4 : 2);
         }
+        // Each scalar update goes from one of the two states to the other where
+        // the kernels finish their reductions themselves (MGFin).  The last one
+        // of a batch is k_finish's, into c->sc for the host.
+        SolverScalars* sc = c->sc;
+        auto fin = [&](int kind, double* part) {
+            MGFin f{kind, grid, part, sc, sc, ctl};
+            if (own && kind >= 0) f.out = sc = sc == c->sc ? c->sc + 1 : c->sc;
+            return f;
+        };
         for (int b = 0; b < batch; ++b) {
             if (first)
-                mg_vcycle<T, 0, true>(c, p, ph);
+                mg_vcycle<T, 0, true, false>(c, fin(-1, nullptr), p, ph);
+            else if (own && b > 0)
+                mg_vcycle<T, 0, false, true>(c, fin(FIN_BETA, part_x), p, ph);
             else
-                mg_vcycle<T, 0, false>(c, p, ph);
+                mg_vcycle<T, 0, false, false>(c, fin(-1, nullptr), p, ph);
             k_mg_v<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, ph,
-                                                          rhat, v, c->part, c->sc);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_ALPHA, grid, c->part, c->sc, ctl);
-            mg_vcycle<T, 1, false>(c, s, sh);
+                                                          rhat, v, c->part, sc);
+            if (own) {
+                mg_vcycle<T, 1, false, true>(c, fin(FIN_ALPHA, c->part), s, sh);
+            } else {
+                k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_ALPHA, grid, c->part, sc, sc, ctl);
+                mg_vcycle<T, 1, false, false>(c, fin(-1, nullptr), s, sh);
+            }
             k_mg_t<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, sh, s,
-                                                          t, c->part, c->sc);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_OMEGA, grid, c->part, c->sc, ctl);
-            k_mg_x<T><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, c->part, c->sc);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, c->part, c->sc, ctl);
+                                                          t, c->part, sc);
+            if (own) {
+                k_mg_x<T, true><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, part_x,
+                                                               fin(FIN_OMEGA, c->part));
+                if (b + 1 == batch)
+                    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, part_x, sc, c->sc, ctl);
+            } else {
+                k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_OMEGA, grid, c->part, sc, sc, ctl);
+                k_mg_x<T, false><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, part_x,
+                                                                fin(-1, nullptr));
+                k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, part_x, sc, sc, ctl);
+            }
             first = false;
         }
         HIPCHK(c, hipGetLastError());
@@ -1548,8 +1644,8 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
     ResidArgs ra = resid_args(c, x, r64, sys.val64, sys.rhs);
     if constexpr (std::is_same<TI, short>::value) ra.nbr16 = nbr;
     k_resid<<<grid, BLOCK, 0, c->stream>>>(ra, 0, nullptr, nullptr);
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_INIT, grid, c->part, c->sc, solve_ctl(c, 0));
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, ctl);
+    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_INIT, grid, c->part, c->sc, c->sc, solve_ctl(c, 0));
+    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, c->sc, ctl);
     HIPCHK(c, hipGetLastError());
     if ((rc = read_sc(c))) return rc;
     if (c->sc_host->done == DONE_ZERO_RHS) {
@@ -1558,7 +1654,7 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
     }
     if (c->sc_host->done == DONE_CONVERGED) return ISPH_OK;
     k_mg_start<true><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4], c->part);
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, ctl);
+    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, c->sc, ctl);
     HIPCHK(c, hipGetLastError());
     if ((rc = read_sc(c))) return rc;
     bool first = true;
@@ -1569,7 +1665,7 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
         if (d != DONE_UPDATE) return fail(c, ISPH_E_STATE, "unexpected solver state");
         k_mx_flush<double><<<nblk(c->n), BLOCK, 0, c->stream>>>(c->n, x, c->v64[4]);
         k_resid<<<grid, BLOCK, 0, c->stream>>>(ra, 0, nullptr, nullptr);
-        k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, ctl_flush);
+        k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, c->sc, ctl_flush);
         HIPCHK(c, hipGetLastError());
         if ((rc = read_sc(c))) return rc;
         if (c->sc_host->done == DONE_CONVERGED) return ISPH_OK;
@@ -1578,12 +1674,12 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
         if (c->sc_host->brk) {
             k_mg_start<true><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4],
                                                             c->part);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, c->sc, ctl);
             first = true;
         } else {
             k_mg_start<false><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4],
                                                              c->part);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_REPLACE, grid, c->part, c->sc, ctl);
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_REPLACE, grid, c->part, c->sc, c->sc, ctl);
         }
         HIPCHK(c, hipGetLastError());
         if ((rc = read_sc(c))) return rc;

@@ -175,11 +175,12 @@ __global__ void __launch_bounds__(BLOCK) k_krylov_3(KrylovArgs<TV, TX, TI> a,
 }
 
 // One block of FIN_BLOCK threads: finish the reductions of the preceding row
-// kernel and update the solver scalars.  Thread t sums partials t,
-// t+FIN_BLOCK, ... in order, then the block tree.
+// kernel and update the solver scalars, from sc into out (which may be sc).
+// Thread t sums partials t, t+FIN_BLOCK, ... in order, then the block tree.
 __global__ void __launch_bounds__(FIN_BLOCK) k_finish(int kind, int nbp,
                                                       const double* __restrict__ part,
-                                                      SolverScalars* sc, SolveCtl ctl) {
+                                                      const SolverScalars* sc, SolverScalars* out,
+                                                      SolveCtl ctl) {
     const bool two = kind != FIN_ALPHA && kind != FIN_START && kind != FIN_REPLACE;
     // The partials and the solver state are loaded before anything waits on
     // either, so neither the done test nor the update below adds its load
@@ -192,7 +193,10 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_finish(int kind, int nbp,
         p1[u] = (two && k < nbp) ? part[nbp + k] : 0.0;
     }
     SolverScalars s = *sc;
-    if ((kind == FIN_ALPHA || kind == FIN_OMEGA || kind == FIN_BETA) && s.done) return;
+    if ((kind == FIN_ALPHA || kind == FIN_OMEGA || kind == FIN_BETA) && s.done) {
+        if (threadIdx.x == 0) *out = s;
+        return;
+    }
     double s0 = 0.0, s1 = 0.0;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -209,7 +213,7 @@ __global__ void __launch_bounds__(FIN_BLOCK) k_finish(int kind, int nbp,
     const double t1 = two ? block_sum_fin(s1) : 0.0;
     if (threadIdx.x != 0) return;
     finish_update(kind, t0, t1, s, ctl);
-    *sc = s;
+    *out = s;
 }
 
 // r = b - A64 x in FP64; partials (b,b), (r,r).  mode 1 also restarts the
