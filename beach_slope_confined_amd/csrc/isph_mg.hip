@@ -42,12 +42,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <vector>
 
 #include "isph_host.h"
 #include "isph_finish.h"
 #include "isph_kernels.h"
+#include "isph_spmv.h"
 
 namespace isph {
 
@@ -55,6 +57,9 @@ constexpr int MG_CMAX = 1024;  // top block level: at most this many cells (one 
 constexpr int MG_CLOW = 768;   // the block's lower levels together: at most this many cells
 constexpr int MG_CLEV = 16;    // at most this many block levels
 constexpr int MG_MAXLEV = 32;  // grid levels in all
+constexpr double MG_RATE0 = 1.0;  // log of an iteration's residual reduction, before any is known
+constexpr int MG_BATCH0 = 4;        // iterations enqueued at once: the first time,
+constexpr int MG_BATCH = 12;        // and at most
 constexpr int MG_BLOCK_NU = 3;      // block levels: sweeps before and after the correction
 // block V-cycles per coarse solve: a deeper block hierarchy compounds the
 // under-correction of its aggregates, so it gets more cycles
@@ -1278,9 +1283,7 @@ __global__ void __launch_bounds__(BLOCK) k_mg_x(int n, const T* __restrict__ ph,
     }
 }
 
-// START: rhat = r, xs = 0, partial (r, r): a first iteration or a restart.
-// Otherwise partial (r, rhat): r replaced by the true residual.
-template <bool START>
+// rhat = r, xs = 0, partial (r, r): a first iteration or a restart
 __global__ void __launch_bounds__(BLOCK) k_mg_start(int n, const double* __restrict__ r,
                                                     double* __restrict__ rhat,
                                                     double* __restrict__ xs,
@@ -1290,14 +1293,73 @@ __global__ void __launch_bounds__(BLOCK) k_mg_start(int n, const double* __restr
     double v = 0.0;
     if (i < n) {
         const double ri = r[i];
-        if (START) {
-            rhat[i] = ri;
-            xs[i] = 0.0;
-        }
-        v = ri * (START ? ri : rhat[i]);
+        rhat[i] = ri;
+        xs[i] = 0.0;
+        v = ri * ri;
     }
     v = block_sum(v);
     if (threadIdx.x == 0) part[lb] = v;
+}
+
+// The reliable update, enqueued after the iterations that are expected to end
+// a segment, before the host knows: each kernel works only if one of them asked
+// for it.  x += xs, xs = 0; r = b - A x with partials (b, b), (r, r), (r, rhat);
+// the stop test, and where the solve goes on without a restart the scalars of
+// the replaced residual.
+__global__ void k_mg_flush(int n, double* __restrict__ x, double* __restrict__ xs,
+                           const SolverScalars* sc) {
+    const int done = sc->done;
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= n || done != DONE_UPDATE) return;
+    x[i] = x[i] + xs[i];
+    xs[i] = 0.0;
+}
+
+template <class TI>
+__global__ void __launch_bounds__(BLOCK) k_mg_resid(ResidArgs a, const TI* __restrict__ nbr,
+                                                    const double* __restrict__ rhat,
+                                                    const SolverScalars* sc) {
+    if (sc->done != DONE_UPDATE) return;
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int i = lb * BLOCK + threadIdx.x;
+    double vb = 0.0, vr = 0.0, vh = 0.0;
+    if (i < a.n) {
+        const double* __restrict__ x = a.x;
+        auto xj = [&](int j) { return x[j]; };
+        const double s = spmv_row<double, double, TI>(i, a.cnt[i], a.dpos[i], nbr, a.val, a.ld,
+                                                      x[i], xj);
+        const double bi = a.b[i];
+        const double r = bi - s;
+        a.r[i] = r;
+        vb = bi * bi;
+        vr = r * r;
+        vh = r * rhat[i];
+    }
+    vb = block_sum(vb);
+    vr = block_sum(vr);
+    vh = block_sum(vh);
+    if (threadIdx.x == 0) {
+        a.part[lb] = vb;
+        a.part[gridDim.x + lb] = vr;
+        a.part[2 * gridDim.x + lb] = vh;
+    }
+}
+
+__global__ void __launch_bounds__(FIN_BLOCK) k_mg_update(int nbp, const double* __restrict__ part,
+                                                         SolverScalars* sc, SolveCtl ctl) {
+    SolverScalars s = *sc;
+    if (s.done != DONE_UPDATE) return;
+    double v[3];  // k_finish's sums
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+        v[u] = 0.0;
+        for (int k = threadIdx.x; k < nbp; k += FIN_BLOCK) v[u] = v[u] + part[(size_t)u * nbp + k];
+        v[u] = block_sum_fin(v[u]);
+    }
+    if (threadIdx.x != 0) return;
+    finish_update(FIN_RESID, v[0], v[1], s, ctl);
+    if (!s.done && !s.brk) finish_update(FIN_REPLACE, v[2], 0.0, s, ctl);
+    *sc = s;
 }
 
 // FP32 values and FP64 row sums of a Jacobi-scaled FP64 matrix in the
@@ -1564,9 +1626,10 @@ static void mg_vcycle(isph_ctx* c, const MGFin& fin, double* bout, T* out) {
                                                        out, sc);
 }
 
+// `batch` iterations
 template <class T, class TI>
-static int mg_iterate(isph_ctx* c, const MGSystem& sys, const TI* nbr, const SolveCtl& ctl,
-                      bool& first) {
+static void mg_iterations(isph_ctx* c, const MGSystem& sys, const TI* nbr, const SolveCtl& ctl,
+                          bool& first, int batch) {
     const T* val = mg_vals<T>(sys);
     const int grid = nblk8(c->n);
     const int n = c->n;
@@ -1577,58 +1640,44 @@ static int mg_iterate(isph_ctx* c, const MGSystem& sys, const TI* nbr, const Sol
     // k_mg_x's partials: apart from k_mg_t's, which its other blocks may be reading
     double* part_x = c->part + 2 * (size_t)grid;
     const bool own = grid <= MG_FIN_MAX;
-    if (int rc = mg_join(c)) return rc;
-    for (;;) {
-        int batch = 4;
-        const SolverScalars& h = *c->sc_host;
-        if (h.nb > 0 && h.rr > 0) {
-            double target = std::max(ctl.tol * h.nb, ctl.delta * h.rupd);
-            const double ratio = std::sqrt(h.rr) / target;
-            batch = ratio > 100.0 ? 8 : (ratio > 3.0 ? 4 : 2);
+    // Each scalar update goes from one of the two states to the other where
+    // the kernels finish their reductions themselves (MGFin).  The last one
+    // of a batch is k_finish's, into c->sc for the host.
+    SolverScalars* sc = c->sc;
+    auto fin = [&](int kind, double* part) {
+        MGFin f{kind, grid, part, sc, sc, ctl};
+        if (own && kind >= 0) f.out = sc = sc == c->sc ? c->sc + 1 : c->sc;
+        return f;
+    };
+    for (int b = 0; b < batch; ++b) {
+        if (first)
+            mg_vcycle<T, 0, true, false>(c, fin(-1, nullptr), p, ph);
+        else if (own && b > 0)
+            mg_vcycle<T, 0, false, true>(c, fin(FIN_BETA, part_x), p, ph);
+        else
+            mg_vcycle<T, 0, false, false>(c, fin(-1, nullptr), p, ph);
+        k_mg_v<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, ph,
+                                                      rhat, v, c->part, sc);
+        if (own) {
+            mg_vcycle<T, 1, false, true>(c, fin(FIN_ALPHA, c->part), s, sh);
+        } else {
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_ALPHA, grid, c->part, sc, sc, ctl);
+            mg_vcycle<T, 1, false, false>(c, fin(-1, nullptr), s, sh);
         }
-        // Each scalar update goes from one of the two states to the other where
-        // the kernels finish their reductions themselves (MGFin).  The last one
-        // of a batch is k_finish's, into c->sc for the host.
-        SolverScalars* sc = c->sc;
-        auto fin = [&](int kind, double* part) {
-            MGFin f{kind, grid, part, sc, sc, ctl};
-            if (own && kind >= 0) f.out = sc = sc == c->sc ? c->sc + 1 : c->sc;
-            return f;
-        };
-        for (int b = 0; b < batch; ++b) {
-            if (first)
-                mg_vcycle<T, 0, true, false>(c, fin(-1, nullptr), p, ph);
-            else if (own && b > 0)
-                mg_vcycle<T, 0, false, true>(c, fin(FIN_BETA, part_x), p, ph);
-            else
-                mg_vcycle<T, 0, false, false>(c, fin(-1, nullptr), p, ph);
-            k_mg_v<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, ph,
-                                                          rhat, v, c->part, sc);
-            if (own) {
-                mg_vcycle<T, 1, false, true>(c, fin(FIN_ALPHA, c->part), s, sh);
-            } else {
-                k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_ALPHA, grid, c->part, sc, sc, ctl);
-                mg_vcycle<T, 1, false, false>(c, fin(-1, nullptr), s, sh);
-            }
-            k_mg_t<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, sh, s,
-                                                          t, c->part, sc);
-            if (own) {
-                k_mg_x<T, true><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, part_x,
-                                                               fin(FIN_OMEGA, c->part));
-                if (b + 1 == batch)
-                    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, part_x, sc, c->sc, ctl);
-            } else {
-                k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_OMEGA, grid, c->part, sc, sc, ctl);
-                k_mg_x<T, false><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, part_x,
-                                                                fin(-1, nullptr));
-                k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, part_x, sc, sc, ctl);
-            }
-            first = false;
+        k_mg_t<TI, T><<<grid, BLOCK, 0, c->stream>>>(n, ld, nbr, c->cnt, val, sys.rsum, sh, s,
+                                                      t, c->part, sc);
+        if (own) {
+            k_mg_x<T, true><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, part_x,
+                                                           fin(FIN_OMEGA, c->part));
+            if (b + 1 == batch)
+                k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, part_x, sc, c->sc, ctl);
+        } else {
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_OMEGA, grid, c->part, sc, sc, ctl);
+            k_mg_x<T, false><<<grid, BLOCK, 0, c->stream>>>(n, ph, s, sh, t, rhat, xs, r, part_x,
+                                                            fin(-1, nullptr));
+            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_BETA, grid, part_x, sc, sc, ctl);
         }
-        HIPCHK(c, hipGetLastError());
-        int rc = read_sc(c);
-        if (rc) return rc;
-        if (c->sc_host->done) return ISPH_OK;
+        first = false;
     }
 }
 
@@ -1653,36 +1702,68 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
         return ISPH_OK;
     }
     if (c->sc_host->done == DONE_CONVERGED) return ISPH_OK;
-    k_mg_start<true><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4], c->part);
-    k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, c->sc, ctl);
-    HIPCHK(c, hipGetLastError());
-    if ((rc = read_sc(c))) return rc;
+    if ((rc = mg_join(c))) return rc;
+    // The host reads the scalars once for each batch of iterations and never to
+    // learn what it can compute: what FIN_START leaves is written here as well.
+    SolverScalars& h = *c->sc_host;
+    auto start = [&] {
+        k_mg_start<<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4], c->part);
+        k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, c->sc, ctl);
+        h.rupd = h.nr;
+        h.done = DONE_RUNNING;
+        h.brk = 0;
+    };
+    auto update = [&] {
+        k_mg_flush<<<nblk(c->n), BLOCK, 0, c->stream>>>(c->n, x, c->v64[4], c->sc);
+        k_mg_resid<TI><<<grid, BLOCK, 0, c->stream>>>(ra, nbr, c->v64[0], c->sc);
+        k_mg_update<<<1, FIN_BLOCK, 0, c->stream>>>(grid, c->part, c->sc, ctl_flush);
+    };
+    start();
     bool first = true;
+    double res = h.nr;            // residual norm now
+    double fell = 0.0, took = 0.0;  // log of the residual's fall so far, and its iterations
     for (;;) {
-        if ((rc = mg_iterate<T, TI>(c, sys, nbr, ctl, first))) return rc;
-        const int d = c->sc_host->done;
-        if (d == DONE_FAILED) return fail(c, ISPH_E_NOCONV, "multigrid PPE solve did not converge");
-        if (d != DONE_UPDATE) return fail(c, ISPH_E_STATE, "unexpected solver state");
-        k_mx_flush<double><<<nblk(c->n), BLOCK, 0, c->stream>>>(c->n, x, c->v64[4]);
-        k_resid<<<grid, BLOCK, 0, c->stream>>>(ra, 0, nullptr, nullptr);
-        k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_RESID, grid, c->part, c->sc, c->sc, ctl_flush);
+        // A batch is the iterations that the segment (to the next reliable
+        // update, or to the tolerance) is expected to take at the mean rate so
+        // far, and the update behind them.  An iteration too many costs its
+        // launches, which do nothing (35 us), one too few a wait of the host
+        // (25 us); batches of 8, 4 and 2 by the residual alone launched 22
+        // iterations for 15 at 2.5k rows and waited 9 times, 134 us a needed
+        // iteration where a kernel chain is 60.
+        const double target = std::max(ctl.tol * h.nb, ctl.delta * h.rupd);
+        const double rate = fell > 0.0 ? fell / took : MG_RATE0;
+        const double left = res > target ? std::log(res / target) / rate : 0.0;
+        const int most = took > 0.0 ? MG_BATCH : MG_BATCH0;
+        const int batch = left < (double)most ? std::max(1, (int)std::ceil(left - 0.25)) : most;
+        const int before = h.total;
+        mg_iterations<T, TI>(c, sys, nbr, ctl, first, batch);
+        const bool tail = batch >= left - 0.25;
+        if (tail) update();
         HIPCHK(c, hipGetLastError());
+        const int nupd = h.nupd;
         if ((rc = read_sc(c))) return rc;
-        if (c->sc_host->done == DONE_CONVERGED) return ISPH_OK;
-        if (c->sc_host->done == DONE_FAILED)
-            return fail(c, ISPH_E_NOCONV, "multigrid PPE solve did not converge");
-        if (c->sc_host->brk) {
-            k_mg_start<true><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4],
-                                                            c->part);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_START, grid, c->part, c->sc, c->sc, ctl);
-            first = true;
-        } else {
-            k_mg_start<false><<<grid, BLOCK, 0, c->stream>>>(c->n, r64, c->v64[0], c->v64[4],
-                                                             c->part);
-            k_finish<<<1, FIN_BLOCK, 0, c->stream>>>(FIN_REPLACE, grid, c->part, c->sc, c->sc, ctl);
+        if (h.done == DONE_UPDATE) {
+            update();
+            HIPCHK(c, hipGetLastError());
+            if ((rc = read_sc(c))) return rc;
         }
-        HIPCHK(c, hipGetLastError());
-        if ((rc = read_sc(c))) return rc;
+        if (h.done == DONE_CONVERGED) return ISPH_OK;
+        if (h.done == DONE_FAILED) return fail(c, ISPH_E_NOCONV, "multigrid PPE solve did not converge");
+        if (h.done != DONE_RUNNING) return fail(c, ISPH_E_STATE, "unexpected solver state");
+        // h.rr: of the last iteration, also where the residual has been replaced
+        const double now = std::sqrt(h.rr);
+        if (h.total > before && now > 0.0) {
+            fell += std::log(res / now);
+            took += h.total - before;
+        }
+        res = now;
+        if (h.nupd > nupd) {
+            res = h.nr;
+            if (h.brk) {
+                start();
+                first = true;
+            }
+        }
     }
 }
 

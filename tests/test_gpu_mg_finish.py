@@ -38,3 +38,19 @@ def test_partials(require_gpu, side, n, iters, digest):
     x = sim.get_field("pressure")
     assert hashlib.sha256(x.tobytes()).hexdigest()[:16] == digest
     sim.close()
+
+
+@pytest.mark.parametrize("maxit", [1, 3, 4, 5, 9])
+def test_iteration_limit(require_gpu, maxit):
+    """The limit holds wherever it falls in the iterations enqueued at once."""
+    cfg = dict(configs.tank_1m(120))
+    cfg["params"] = cfg["params"].copy(precision=PREC_MIXED_MG, tol=1e-9, maxit=maxit)
+    sim = configs.make_sim(cfg, capi.IsphSim)
+    s = sim.scalars()
+    sim.set_scalars(s["umax"], s["dt"], s["t"] + s["dt"])
+    for st in PRE:
+        getattr(sim, st)()
+    with pytest.raises(capi.IsphError, match="NOCONV"):
+        sim.ppesolve()
+    assert sim.scalars()["iters"] == maxit
+    sim.close()
