@@ -2,6 +2,7 @@
 // (cooperative launches).  Worker blocks publish their part of a sum; one more
 // block, the leader, reads all parts, finishes the reduction and broadcasts
 // what the workers need of it.  The exchange is reduction and barrier in one.
+// Small grids do without the leader: every block reads all parts.
 //
 // Every published 64-bit word carries 32 bits of data under a 32-bit epoch
 // number, so it is valid by itself and no flag has to follow the data.  Words
@@ -9,7 +10,8 @@
 // private L2 caches.  Two buffers alternate by epoch: a worker publishes epoch
 // e + 2 only after the broadcast of e + 1, for which the leader needed every
 // worker's part of e + 1, and a worker publishes that after it has read the
-// broadcast of e; likewise for the leader's words.  The words are zeroed
+// broadcast of e, or without a leader all parts of e; likewise for the
+// leader's words.  The words are zeroed
 // before each launch and epochs count from 1.
 //
 // Vector entries that other blocks read after an exchange are stored with

@@ -26,12 +26,13 @@
 // only where a thread has 128 registers (blocks of 1024 rows) a few stay in
 // memory.
 //
-// What bounds it: the chain of three exchanges (2.3 us each: the words' way to
-// the leader and back, the sums on either side), then two products (0.5 us),
-// the halo reads (0.4 us) and the wait for the stores.  Measured per
-// iteration, launched kernels and here: 30 and 10.3 us at 36.6k rows, 32 and
-// 11.7 us at 87k, 44 and 19 us at 255k.  Values and places in LDS instead of
-// registers, with the diagonal tested at every entry, made a product 1.3 us.
+// What bounds it: the chain of three exchanges (1.3 us each without a leader,
+// 2.3 with one: the words' way, the sums on either side), then two products
+// (0.5 us), the halo reads (0.4 us) and the wait for the stores.  Measured per
+// iteration, launched kernels and here: 29 and 7.4 us at 2.5k rows, 30 and
+// 10.1 us at 36.6k, 32 and 11.4 us at 86k, 44 and 19 us at 255k.  Values and
+// places in LDS instead of registers, with the diagonal tested at every entry,
+// made a product 1.3 us.
 //
 // The arithmetic is the launched kernels', term for term: the same row sums,
 // the same reduction tree (wave butterfly, four waves of 256 rows, then
@@ -212,38 +213,45 @@ __device__ __forceinline__ void publish_sums(const GridSync& gs, double (*wsum)[
     }
 }
 
+// k_finish's sum of the parts of an exchange in one wave.  Lane l takes the
+// parts l + 64 m.  64 / G parts are a wave of k_finish's tree, so the sum over
+// the lanes of one m covers G of its waves, in its order: the butterfly's last
+// log2(G) steps are the first levels of the tree over the waves.
+template <int NP>
+struct PartSums {
+    double a[NP], b[NP];
+    __device__ __forceinline__ bool collect(const GridSync& gs, uint32_t e, int nw, bool two) {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int m = 0; m < NP; ++m) a[m] = b[m] = 0.0;
+        const bool ok = lane >= nw || gs_collect<NP>(gs, e, lane, 64, nw, two, a, b);
+        return __all(ok);
+    }
+    static __device__ __forceinline__ double total(const double* p) {
+        double q[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int m = 0; m < NP; ++m) q[m] = lanes_sum<64>(p[m]);
+        return ((q[0] + q[1]) + (q[2] + q[3])) + 0.0;  // k_finish's remaining waves are 0
+    }
+};
+
 // The leader, one wave: finishes each exchange's reduction and the solver
-// scalars, and broadcasts the scalar that the workers wait for.  Lane l takes
-// the parts l + 64 m.  64 / G parts are a wave of k_finish's tree, so the sum
-// over the lanes of one m covers G of its waves, in its order: the butterfly's
-// last log2(G) steps are the first levels of the tree over the waves.
-template <int G>
+// scalars, and broadcasts the scalar that the workers wait for.
 __device__ __forceinline__ void resident_leader(const GridSync& gs, int nw, SolverScalars* sc,
                                                 const SolveCtl& ctl, int maxiter) {
-    constexpr int NP = GS_MAXB / 64;
     const int t = threadIdx.x;
     if (t >= 64) return;
     SolverScalars s = *sc;
-    double a[NP] = {}, b[NP] = {};
+    PartSums<GS_MAXB / 64> sum;
     auto collect = [&](uint32_t e, bool two) {
-        const bool ok = t >= nw || gs_collect<NP>(gs, e, t, 64, nw, two, a, b);
-        if (!__all(ok)) {
-            if (t == 0) atomicOr(gs.err, ERR_SYNC);
-            return false;
-        }
-        return true;
-    };
-    // k_finish's remaining waves are 0
-    auto total = [](const double* p) {
-        double q[NP];
-#pragma unroll
-        for (int m = 0; m < NP; ++m) q[m] = lanes_sum<64>(p[m]);
-        return ((q[0] + q[1]) + (q[2] + q[3])) + 0.0;
+        const bool ok = sum.collect(gs, e, nw, two);
+        if (!ok && t == 0) atomicOr(gs.err, ERR_SYNC);
+        return ok;
     };
     // epoch 1: do all blocks' windows fit?
     uint32_t e = 1;
     if (!collect(e, false)) return;
-    const int refused = total(a) != 0.0;
+    const int refused = sum.total(sum.a) != 0.0;
     gs_broadcast(gs, e, 0.0, refused);
     if (refused) {
         if (t == 0) atomicOr(gs.state, GS_REFUSED);
@@ -251,20 +259,24 @@ __device__ __forceinline__ void resident_leader(const GridSync& gs, int nw, Solv
     }
     for (int it = 0; it < maxiter; ++it) {
         if (!collect(++e, false)) return;
-        finish_update(FIN_ALPHA, total(a), 0.0, s, ctl);
+        finish_update(FIN_ALPHA, sum.total(sum.a), 0.0, s, ctl);
         gs_broadcast(gs, e, s.alpha, 0);
         if (!collect(++e, true)) return;
-        finish_update(FIN_OMEGA, total(a), total(b), s, ctl);
+        finish_update(FIN_OMEGA, sum.total(sum.a), sum.total(sum.b), s, ctl);
         gs_broadcast(gs, e, s.wi, 0);
         if (!collect(++e, true)) return;
-        finish_update(FIN_BETA, total(a), total(b), s, ctl);
+        finish_update(FIN_BETA, sum.total(sum.a), sum.total(sum.b), s, ctl);
         gs_broadcast(gs, e, s.betas, s.done);
         if (s.done) break;
     }
     if (t == 0) *sc = s;
 }
 
-template <class TV, class TX, int G>
+// NP > 0: no leader; one wave of every block sums all parts, up to 64 NP, and
+// forms the scalars.  The words travel once instead of to the leader and back;
+// what grows with the grid is the reading of all parts by all blocks.  (Four
+// waves a block that read a quarter each, or all, are slower at any size.)
+template <class TV, class TX, int G, int NP>
 __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, short> a, GridSync gs,
                                                              SolverScalars* sc, SolveCtl ctl,
                                                              int first, int maxiter,
@@ -278,9 +290,9 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
     __shared__ double sums[2][16];
     __shared__ Window W;
     __shared__ int jlo, jhi, total;
-    const int nw = gridDim.x - 1;
-    if ((int)blockIdx.x == nw) {
-        resident_leader<G>(gs, nw, sc, ctl, maxiter);
+    const int nw = NP ? gridDim.x : gridDim.x - 1;
+    if (!NP && (int)blockIdx.x == nw) {
+        resident_leader(gs, nw, sc, ctl, maxiter);
         return;
     }
     const int block = xcd_tile(blockIdx.x, nw);
@@ -343,12 +355,42 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
     uint32_t e = 1;
     double coef = 0.0;
     int done = 0;
+    __shared__ double answer[2];  // NP: the awaited scalar; the stop flag, or -1
+    SolverScalars s;
+    if (NP) s = *sc;
+    auto exchanged = [&](int kind) {
+        if (!NP) return gs_receive(gs, e, block, coef, done);
+        if (t < 64) {
+            PartSums<NP ? NP : 1> sum;
+            const bool two = kind == FIN_OMEGA || kind == FIN_BETA;
+            const bool ok = sum.collect(gs, e, nw, two);
+            const double t0 = sum.total(sum.a);
+            if (kind < 0) {
+                done = t0 != 0.0;
+            } else {
+                finish_update(kind, t0, two ? sum.total(sum.b) : 0.0, s, ctl);
+                coef = kind == FIN_ALPHA ? s.alpha : kind == FIN_OMEGA ? s.wi : s.betas;
+                done = kind == FIN_BETA ? s.done : 0;
+            }
+            if (t == 0) {
+                answer[0] = coef;
+                answer[1] = ok ? (double)done : -1.0;
+            }
+        }
+        __syncthreads();  // the next exchange's, in publish_sums, orders the reads
+        coef = answer[0];
+        done = (int)answer[1];
+        return done >= 0;
+    };
     if (t == 0) gs_publish(gs, e, block, false, fits ? 0.0 : 1.0, 0.0);
-    if (!gs_receive(gs, e, block, coef, done)) {
+    if (!exchanged(-1)) {
         atomicOr(gs.err, ERR_SYNC);
         return;
     }
-    if (done) return;  // some block's window does not fit
+    if (done) {  // some block's window does not fit
+        if (NP && block == 0 && t == 0) atomicOr(gs.state, GS_REFUSED);
+        return;
+    }
     const int nh = total - nown, nl = W.place(i0 - base);
     TX* win = reinterpret_cast<TX*>(dyn);
     TV* lv = reinterpret_cast<TV*>(win + (M + 1) * R) + t;
@@ -418,7 +460,7 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         }
         publish_sums<G, false, true>(gs, sums, ++e, block, own ? (double)v * (double)rhat : 0.0,
                                      0.0);
-        if (!(ok = gs_receive(gs, e, block, coef, done))) break;
+        if (!(ok = exchanged(FIN_ALPHA))) break;
         // s = r - alpha v, t = A s
         const TX alpha = (TX)coef;
         const TX sv = r - alpha * v;
@@ -440,7 +482,7 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         }
         publish_sums<G, true, true>(gs, sums, ++e, block, own ? (double)tv * (double)sv : 0.0,
                                     own ? (double)tv * (double)tv : 0.0);
-        if (!(ok = gs_receive(gs, e, block, coef, done))) break;
+        if (!(ok = exchanged(FIN_OMEGA))) break;
         // x, r, q
         const TX w = (TX)coef;
         TX ht[M];
@@ -452,7 +494,7 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         q = p - w * v;
         publish_sums<G, true, false>(gs, sums, ++e, block, own ? (double)r * (double)rhat : 0.0,
                                      own ? (double)r * (double)r : 0.0);
-        if (!(ok = gs_receive(gs, e, block, coef, done))) break;
+        if (!(ok = exchanged(FIN_BETA))) break;
         if (done) break;
         // the halo rows' t arrived while the block waited
 #pragma unroll
@@ -466,6 +508,7 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         return;
     }
     if (t == 0) atomicOr(gs.state, GS_WRITTEN);
+    if (NP && block == 0 && t == 0) *sc = s;
     if (own) {
         a.xs[i] = x;
         P2 u;
@@ -477,12 +520,12 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
 
 namespace host {
 
-template <class TV, class TX, int G>
+template <class TV, class TX, int G, int NP>
 static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveCtl& ctl, bool& first,
                   int maxiter, bool& ran) {
-    auto kern = k_bicg_resident<TV, TX, G>;
+    auto kern = k_bicg_resident<TV, TX, G, NP>;
     constexpr int R = BLOCK * G;
-    const int blocks = (nblk(c->n) + G - 1) / G + 1;
+    const int blocks = (nblk(c->n) + G - 1) / G + (NP ? 0 : 1);
     if (blocks > c->cus) return ISPH_OK;
     // the gathered window, then as many of each row's further entries as fit
     constexpr size_t win = sizeof(TX) * (RESIDENT_M + 1) * R;
@@ -503,16 +546,21 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
 
 // Rows per block, 256 G: as few as let the grid hold the system with one
 // worker per CU and a CU for the leader: G = 1 up to 65,280 rows, 2 up to
-// 130,560, 4 up to 261,120.
+// 130,560, 4 up to 261,120.  Up to 160 blocks exchange without a leader: an
+// iteration takes 7.4 us against 10.4 at 10 blocks, 7.8 / 9.6 at 43, 9.2 / 10.1
+// at 70, 10.1 / 10.9 at 144, but 10.8 / 10.4 at 185, where every block's reading
+// of every part costs more than the leader's round trip.
 template <class TV, class TX>
 int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
                      bool& first, int maxiter, bool& ran) {
     ran = false;
     if (!c->cooperative || c->n == 0) return ISPH_OK;
     const int nb = nblk(c->n), most = GS_MAXB - 1;
-    if (nb <= most) return launch<TV, TX, 1>(c, a, ctl, first, maxiter, ran);
-    if (nb <= 2 * most) return launch<TV, TX, 2>(c, a, ctl, first, maxiter, ran);
-    if (nb <= 4 * most) return launch<TV, TX, 4>(c, a, ctl, first, maxiter, ran);
+    if (nb <= 64) return launch<TV, TX, 1, 1>(c, a, ctl, first, maxiter, ran);
+    if (nb <= 160) return launch<TV, TX, 1, 3>(c, a, ctl, first, maxiter, ran);
+    if (nb <= most) return launch<TV, TX, 1, 0>(c, a, ctl, first, maxiter, ran);
+    if (nb <= 2 * most) return launch<TV, TX, 2, 0>(c, a, ctl, first, maxiter, ran);
+    if (nb <= 4 * most) return launch<TV, TX, 4, 0>(c, a, ctl, first, maxiter, ran);
     return streamed_iterate<TV, TX>(c, a, ctl, first, maxiter, ran);
 }
 
