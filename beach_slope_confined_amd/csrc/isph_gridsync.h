@@ -87,12 +87,22 @@ __device__ __forceinline__ void gs_publish(const GridSync& g, uint32_t e, int pa
     }
 }
 
+// Words that a thread waits for besides an exchange's: they are requested with
+// every poll, and the wait goes on until they are valid too.
+struct GsNone {
+    __device__ __forceinline__ void request() {}
+    __device__ __forceinline__ bool valid() const { return true; }
+    __device__ __forceinline__ bool wait() { return true; }
+};
+
 // leader: a thread reads the N parts first, first + stride, .. of epoch e that
 // lie below `count` (the others are 0); false if one did not come
-template <int N>
+template <int N, class More>
 __device__ __forceinline__ bool gs_collect(const GridSync& g, uint32_t e, int first, int stride,
-                                           int count, bool two, double* v0, double* v1) {
+                                           int count, bool two, double* v0, double* v1,
+                                           More& more) {
     for (int spin = 0; spin < GS_SPIN; ++spin) {
+        more.request();
         gs_word x[N][4];
 #pragma unroll
         for (int m = 0; m < N; ++m) {
@@ -102,7 +112,7 @@ __device__ __forceinline__ bool gs_collect(const GridSync& g, uint32_t e, int fi
             for (int q = 0; q < 4; ++q)
                 x[m][q] = in && (q < 2 || two) ? gs_load(w + q * g.parts) : (gs_word)e << 32;
         }
-        bool ok = true;
+        bool ok = more.valid();
 #pragma unroll
         for (int m = 0; m < N; ++m)
 #pragma unroll
@@ -117,6 +127,13 @@ __device__ __forceinline__ bool gs_collect(const GridSync& g, uint32_t e, int fi
         }
     }
     return false;
+}
+
+template <int N>
+__device__ __forceinline__ bool gs_collect(const GridSync& g, uint32_t e, int first, int stride,
+                                           int count, bool two, double* v0, double* v1) {
+    GsNone none;
+    return gs_collect<N>(g, e, first, stride, count, two, v0, v1, none);
 }
 
 // leader: threads 0 .. GS_LINES - 1 broadcast a value and a flag
@@ -147,5 +164,4 @@ __device__ __forceinline__ bool gs_receive(const GridSync& g, uint32_t e, int bl
     }
     return false;
 }
-
 }  // namespace isph

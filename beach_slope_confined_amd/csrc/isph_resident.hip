@@ -12,7 +12,7 @@
 // window; a bitmap of them gives a row's place in it.
 //
 //   p = r + beta q, v = A p               own and halo p into LDS, product
-//     exchange (v, rhat) -> alpha         v of the halo rows is read after it
+//     exchange (v, rhat) -> alpha         v of the halo rows is read with it
 //   s = r - alpha v, t = A s              own and halo s into LDS, product
 //     exchange (t, s), (t, t) -> omega    t of the halo rows is read after it
 //   x += alpha p + omega s, r = s - omega t, q = p - omega v   own and halo
@@ -28,11 +28,11 @@
 //
 // What bounds it: the chain of three exchanges (1.3 us each without a leader,
 // 2.3 with one: the words' way, the sums on either side), then two products
-// (0.5 us), the halo reads (0.4 us) and the wait for the stores.  Measured per
-// iteration, launched kernels and here: 29 and 7.4 us at 2.5k rows, 30 and
-// 10.1 us at 36.6k, 32 and 11.4 us at 86k, 44 and 19 us at 255k.  Values and
-// places in LDS instead of registers, with the diagonal tested at every entry,
-// made a product 1.3 us.
+// (0.5 us), and with a leader the halo reads (0.4 us) and the wait for the
+// stores.  Measured per iteration, launched kernels and here: 29 and 7.0 us at
+// 2.5k rows, 30 and 9.0 us at 36.6k, 32 and 11.4 us at 86k, 44 and 19 us at
+// 255k.  Values and places in LDS instead of registers, with the diagonal
+// tested at every entry, made a product 1.3 us.
 //
 // The arithmetic is the launched kernels', term for term: the same row sums,
 // the same reduction tree (wave butterfly, four waves of 256 rows, then
@@ -180,8 +180,81 @@ struct ResidentRow {
     }
 };
 
+// Without a leader, vector entries that other blocks read are 64-bit words of
+// 32 bits of data under the epoch, like the exchanges' (an FP64 value takes
+// two), so that neither the writer waits for its stores before it publishes its
+// part of the sum, nor the reader for the sum before it asks for them.  A word
+// is written again three epochs later, when its writer has seen every block's
+// part of an epoch that the block published after it had read the word.
+// Cleared before each launch.  8.2 against 9.2 us an iteration at 17.7k rows;
+// with a leader (the workers' polls of its words and of these then compete) it
+// is no faster at 59k and 86k rows, and blocks of 1024 rows lack the registers
+// (24.6 against 19.4 us at 255k), so there the entries are plain.
+struct HaloWords {
+    gs_word *vh, *vl, *th, *tl;  // high and low words of v and t
+};
+// 32-bit byte offsets: one register an address
+__device__ __forceinline__ gs_word* word_at(gs_word* w, int j) {
+    return reinterpret_cast<gs_word*>(reinterpret_cast<char*>(w) + (unsigned int)j * 8u);
+}
+__device__ __forceinline__ void store_words(gs_word* h, gs_word* l, int i, uint32_t e, double v) {
+    gs_store(word_at(h, i), gs_hi(e, v));
+    gs_store(word_at(l, i), gs_lo(e, v));
+}
+__device__ __forceinline__ void store_words(gs_word* h, gs_word*, int i, uint32_t e, float v) {
+    gs_store(word_at(h, i), (gs_word)e << 32 | __float_as_uint(v));
+}
+template <class TX>
+struct HaloRead {
+    static constexpr bool WIDE = sizeof(TX) == 8;
+    gs_word *h, *l;
+    const int* row;  // M of them, -1 for none
+    uint32_t e;
+    gs_word x[RESIDENT_M], y[RESIDENT_M];
+    __device__ __forceinline__ void request() {
+#pragma unroll
+        for (int m = 0; m < RESIDENT_M; ++m) {
+            x[m] = y[m] = (gs_word)e << 32;
+            if (row[m] >= 0) {
+                x[m] = gs_load(word_at(h, row[m]));
+                if (WIDE) y[m] = gs_load(word_at(l, row[m]));
+            }
+        }
+    }
+    __device__ __forceinline__ bool valid() const {
+        bool ok = true;
+#pragma unroll
+        for (int m = 0; m < RESIDENT_M; ++m)
+            ok = ok && (uint32_t)(x[m] >> 32) == e && (!WIDE || (uint32_t)(y[m] >> 32) == e);
+        return ok;
+    }
+    __device__ __forceinline__ TX value(int m) const {
+        if constexpr (WIDE) return gs_value(x[m], y[m]);
+        else return __uint_as_float((unsigned int)x[m]);
+    }
+    // a wave that waits for nothing else
+    __device__ __forceinline__ bool wait() {
+        for (int spin = 0; spin < GS_SPIN; ++spin) {
+            request();
+            if (__all(valid())) return true;
+        }
+        return false;
+    }
+};
+
+__global__ void k_halo_clear(int n, HaloWords w, bool wide) {
+    const int i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= n) return;
+    w.vh[i] = 0ull;
+    w.th[i] = 0ull;
+    if (wide) {
+        w.vl[i] = 0ull;
+        w.tl[i] = 0ull;
+    }
+}
+
 // A worker's part of an exchange: the block's partials in the launched
-// kernels' tree, published by one thread.  STORED: the waves have stored
+// kernels' tree, published by one thread.  STORED: the waves have stored plain
 // vector entries that others read after the exchange; vmcnt counts stores on
 // this architecture, so each wave waits for its own before the block's barrier.
 template <int G, bool TWO, bool STORED>
@@ -220,12 +293,11 @@ __device__ __forceinline__ void publish_sums(const GridSync& gs, double (*wsum)[
 template <int NP>
 struct PartSums {
     double a[NP], b[NP];
-    __device__ __forceinline__ bool collect(const GridSync& gs, uint32_t e, int nw, bool two) {
+    template <class More>
+    __device__ __forceinline__ bool collect(const GridSync& gs, uint32_t e, int nw, bool two,
+                                            More& more) {
         const int lane = threadIdx.x & 63;
-#pragma unroll
-        for (int m = 0; m < NP; ++m) a[m] = b[m] = 0.0;
-        const bool ok = lane >= nw || gs_collect<NP>(gs, e, lane, 64, nw, two, a, b);
-        return __all(ok);
+        return __all(gs_collect<NP>(gs, e, lane, 64, nw, two, a, b, more));
     }
     static __device__ __forceinline__ double total(const double* p) {
         double q[4] = {0.0, 0.0, 0.0, 0.0};
@@ -244,7 +316,8 @@ __device__ __forceinline__ void resident_leader(const GridSync& gs, int nw, Solv
     SolverScalars s = *sc;
     PartSums<GS_MAXB / 64> sum;
     auto collect = [&](uint32_t e, bool two) {
-        const bool ok = sum.collect(gs, e, nw, two);
+        GsNone none;
+        const bool ok = sum.collect(gs, e, nw, two, none);
         if (!ok && t == 0) atomicOr(gs.err, ERR_SYNC);
         return ok;
     };
@@ -279,8 +352,8 @@ __device__ __forceinline__ void resident_leader(const GridSync& gs, int nw, Solv
 template <class TV, class TX, int G, int NP>
 __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, short> a, GridSync gs,
                                                              SolverScalars* sc, SolveCtl ctl,
-                                                             int first, int maxiter,
-                                                             int kl) {
+                                                             HaloWords words, int first,
+                                                             int maxiter, int kl) {
     using P2 = typename Pair2<TX>::type;
     constexpr bool DIFF = std::is_same<TV, float>::value && std::is_same<TX, double>::value;
     constexpr int R = BLOCK * G;
@@ -358,12 +431,13 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
     __shared__ double answer[2];  // NP: the awaited scalar; the stop flag, or -1
     SolverScalars s;
     if (NP) s = *sc;
-    auto exchanged = [&](int kind) {
+    auto exchanged = [&](int kind, auto& more) {
         if (!NP) return gs_receive(gs, e, block, coef, done);
+        bool ok;
         if (t < 64) {
             PartSums<NP ? NP : 1> sum;
             const bool two = kind == FIN_OMEGA || kind == FIN_BETA;
-            const bool ok = sum.collect(gs, e, nw, two);
+            ok = sum.collect(gs, e, nw, two, more);
             const double t0 = sum.total(sum.a);
             if (kind < 0) {
                 done = t0 != 0.0;
@@ -376,14 +450,17 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
                 answer[0] = coef;
                 answer[1] = ok ? (double)done : -1.0;
             }
+        } else {
+            ok = more.wait();
         }
         __syncthreads();  // the next exchange's, in publish_sums, orders the reads
         coef = answer[0];
         done = (int)answer[1];
-        return done >= 0;
+        return ok && done >= 0;
     };
+    GsNone none;
     if (t == 0) gs_publish(gs, e, block, false, fits ? 0.0 : 1.0, 0.0);
-    if (!exchanged(-1)) {
+    if (!exchanged(-1, none)) {
         atomicOr(gs.err, ERR_SYNC);
         return;
     }
@@ -456,18 +533,19 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         TX v = (TX)0;
         if (own) {
             v = row.times(a, W, base, kl, win, p);
-            gs_store(at(vout, i), v);
+            if (NP) store_words(words.vh, words.vl, i, e + 1, v);
+            else gs_store(at(vout, i), v);
         }
-        publish_sums<G, false, true>(gs, sums, ++e, block, own ? (double)v * (double)rhat : 0.0,
-                                     0.0);
-        if (!(ok = exchanged(FIN_ALPHA))) break;
+        publish_sums<G, false, !NP>(gs, sums, ++e, block, own ? (double)v * (double)rhat : 0.0, 0.0);
+        HaloRead<TX> rv{words.vh, words.vl, hj, e};
+        if (!(ok = exchanged(FIN_ALPHA, rv))) break;
         // s = r - alpha v, t = A s
         const TX alpha = (TX)coef;
         const TX sv = r - alpha * v;
         if (own) win[nl + t] = sv;
 #pragma unroll
         for (int m = 0; m < M; ++m)
-            if (hj[m] >= 0) hv[m] = gs_load(at(vout, hj[m]));
+            if (hj[m] >= 0) hv[m] = NP ? rv.value(m) : gs_load(at(vout, hj[m]));
 #pragma unroll
         for (int m = 0; m < M; ++m)
             if (hj[m] >= 0) {
@@ -478,28 +556,30 @@ __global__ void __launch_bounds__(BLOCK* G) k_bicg_resident(KrylovArgs<TV, TX, s
         TX tv = (TX)0;
         if (own) {
             tv = row.times(a, W, base, kl, win, sv);
-            gs_store(at(tout, i), tv);
+            if (NP) store_words(words.th, words.tl, i, e + 1, tv);
+            else gs_store(at(tout, i), tv);
         }
-        publish_sums<G, true, true>(gs, sums, ++e, block, own ? (double)tv * (double)sv : 0.0,
-                                    own ? (double)tv * (double)tv : 0.0);
-        if (!(ok = exchanged(FIN_OMEGA))) break;
+        publish_sums<G, true, !NP>(gs, sums, ++e, block, own ? (double)tv * (double)sv : 0.0,
+                                   own ? (double)tv * (double)tv : 0.0);
+        HaloRead<TX> rt{words.th, words.tl, hj, e};
+        if (!(ok = exchanged(FIN_OMEGA, none))) break;
         // x, r, q
         const TX w = (TX)coef;
         TX ht[M];
 #pragma unroll
         for (int m = 0; m < M; ++m)
-            ht[m] = hj[m] >= 0 ? gs_load(at(tout, hj[m])) : (TX)0;
+            ht[m] = !NP && hj[m] >= 0 ? gs_load(at(tout, hj[m])) : (TX)0;
         x = (x + alpha * p) + w * sv;
         r = sv - w * tv;
         q = p - w * v;
         publish_sums<G, true, false>(gs, sums, ++e, block, own ? (double)r * (double)rhat : 0.0,
                                      own ? (double)r * (double)r : 0.0);
-        if (!(ok = exchanged(FIN_BETA))) break;
+        if (!(ok = exchanged(FIN_BETA, rt))) break;
         if (done) break;
         // the halo rows' t arrived while the block waited
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            hr[m] = hs[m] - w * ht[m];
+            hr[m] = hs[m] - w * (NP ? rt.value(m) : ht[m]);
             hq[m] = hp[m] - w * hv[m];
         }
     }
@@ -537,8 +617,12 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
     GridSync gs{c->gs_words, c->err, c->err + 1, GS_MAXB};
     SolverScalars* sc = c->sc;
     SolveCtl t = ctl;
+    // vectors that the launched kernels write before they read
+    auto words = [](void* p) { return static_cast<gs_word*>(p); };
+    HaloWords h{words(c->rv64), words(c->rv64) + c->cap, words(c->v64[2]), words(c->v64[3])};
+    if (NP) k_halo_clear<<<nblk(c->n), BLOCK, 0, c->stream>>>(c->n, h, sizeof(TX) == 8);
     int f = first, m = maxiter, l = kl;
-    void* args[] = {&a, &gs, &sc, &t, &f, &m, &l};
+    void* args[] = {&a, &gs, &sc, &t, &h, &f, &m, &l};
     if (int rc = grid_launch(c, (const void*)kern, blocks, R, args, lds, GS_MAXB, ran)) return rc;
     if (ran) first = false;
     return ISPH_OK;
@@ -547,8 +631,8 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
 // Rows per block, 256 G: as few as let the grid hold the system with one
 // worker per CU and a CU for the leader: G = 1 up to 65,280 rows, 2 up to
 // 130,560, 4 up to 261,120.  Up to 160 blocks exchange without a leader: an
-// iteration takes 7.4 us against 10.4 at 10 blocks, 7.8 / 9.6 at 43, 9.2 / 10.1
-// at 70, 10.1 / 10.9 at 144, but 10.8 / 10.4 at 185, where every block's reading
+// iteration takes 7.0 us against 10.4 at 10 blocks, 6.9 / 9.6 at 43, 8.2 / 10.1
+// at 70, 9.0 / 10.9 at 144, but 10.5 / 10.4 at 185, where every block's reading
 // of every part costs more than the leader's round trip.
 template <class TV, class TX>
 int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
