@@ -29,8 +29,8 @@
 // What bounds it: the chain of three exchanges (1.3 us each without a leader,
 // 2.3 with one: the words' way, the sums on either side), then two products
 // (0.5 us), and with a leader the halo reads (0.4 us) and the wait for the
-// stores.  Measured per iteration, launched kernels and here: 29 and 7.0 us at
-// 2.5k rows, 30 and 9.0 us at 36.6k, 32 and 11.4 us at 86k, 44 and 19 us at
+// stores.  Measured per iteration, launched kernels and here: 29 and 6.9 us at
+// 2.5k rows, 30 and 7.9 us at 36.6k, 32 and 9.7 us at 86k, 44 and 19 us at
 // 255k.  Values and places in LDS instead of registers, with the diagonal
 // tested at every entry, made a product 1.3 us.
 //
@@ -186,10 +186,10 @@ struct ResidentRow {
 // part of the sum, nor the reader for the sum before it asks for them.  A word
 // is written again three epochs later, when its writer has seen every block's
 // part of an epoch that the block published after it had read the word.
-// Cleared before each launch.  8.2 against 9.2 us an iteration at 17.7k rows;
-// with a leader (the workers' polls of its words and of these then compete) it
-// is no faster at 59k and 86k rows, and blocks of 1024 rows lack the registers
-// (24.6 against 19.4 us at 255k), so there the entries are plain.
+// Cleared before each launch.  8.2 against 9.2 us an iteration at 17.7k rows in
+// blocks of 256; with a leader (the workers' polls of its words and of these
+// then compete) it is no faster at 59k and 86k rows, and blocks of 1024 rows
+// lack the registers (24.6 against 19.4 us at 255k), so there they are plain.
 struct HaloWords {
     gs_word *vh, *vl, *th, *tl;  // high and low words of v and t
 };
@@ -628,12 +628,15 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
     return ISPH_OK;
 }
 
-// Rows per block, 256 G: as few as let the grid hold the system with one
-// worker per CU and a CU for the leader: G = 1 up to 65,280 rows, 2 up to
-// 130,560, 4 up to 261,120.  Up to 160 blocks exchange without a leader: an
-// iteration takes 7.0 us against 10.4 at 10 blocks, 6.9 / 9.6 at 43, 8.2 / 10.1
-// at 70, 9.0 / 10.9 at 144, but 10.5 / 10.4 at 185, where every block's reading
-// of every part costs more than the leader's round trip.
+// Rows per block, 256 G, and whether a leader serves the exchanges.  Up to 192
+// blocks do without (NP parts a lane): the words' round trip saved is more than
+// every block's reading of every part, and so fewer, larger blocks are better
+// from 64 on.  Measured with blocks of 256 and of 512 rows: 6.9 and 6.95 us an
+// iteration at 11k rows, 7.8 / 7.0 at 17.7k, 9.1 / 7.9 at 36.6k, 9.7 / 8.1 at
+// 47k; with and without a leader 11.6 / 8.2 at 59k, 10.8 / 9.4 at 72.5k, 10.9 /
+// 9.7 at 86k, but 11.5 / 13.4 at 103k.  Beyond 98k rows a leader, and beyond
+// 130,560 blocks of 1024 rows, as few as let the grid hold the system with one
+// worker per CU and a CU for the leader, up to 261,120.
 template <class TV, class TX>
 int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
                      bool& first, int maxiter, bool& ran) {
@@ -641,8 +644,9 @@ int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const Solv
     if (!c->cooperative || c->n == 0) return ISPH_OK;
     const int nb = nblk(c->n), most = GS_MAXB - 1;
     if (nb <= 64) return launch<TV, TX, 1, 1>(c, a, ctl, first, maxiter, ran);
-    if (nb <= 160) return launch<TV, TX, 1, 3>(c, a, ctl, first, maxiter, ran);
-    if (nb <= most) return launch<TV, TX, 1, 0>(c, a, ctl, first, maxiter, ran);
+    if (nb <= 128) return launch<TV, TX, 2, 1>(c, a, ctl, first, maxiter, ran);
+    if (nb <= 256) return launch<TV, TX, 2, 2>(c, a, ctl, first, maxiter, ran);
+    if (nb <= 384) return launch<TV, TX, 2, 3>(c, a, ctl, first, maxiter, ran);
     if (nb <= 2 * most) return launch<TV, TX, 2, 0>(c, a, ctl, first, maxiter, ran);
     if (nb <= 4 * most) return launch<TV, TX, 4, 0>(c, a, ctl, first, maxiter, ran);
     return streamed_iterate<TV, TX>(c, a, ctl, first, maxiter, ran);
