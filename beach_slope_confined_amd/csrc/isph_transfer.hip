@@ -79,7 +79,21 @@ int download(isph_ctx* c, int64_t rows, const Column* cols, int ncol) {
     if (!pool && hipHostMalloc((void**)&pool, SLOTS * SLOT_BYTES, hipHostMallocPortable) != hipSuccess) {
         pool = nullptr;
         (void)hipGetLastError();
-        return fail(c, ISPH_E_HIP, "no pinned memory for the transfer");
+    }
+    if (!pool) {  // no pinned memory: through the runtime's own staging
+        std::vector<char> t;
+        for (int k = 0; k < ncol; ++k) {
+            const Column& q = cols[k];
+            const bool dense = q.stride == q.size;
+            const size_t len = (size_t)(rows - 1) * q.stride + q.size;
+            if (!dense) t.resize(len);
+            HIPCHK(c, hipMemcpyAsync(dense ? q.dst : t.data(), q.src, len, hipMemcpyDeviceToHost,
+                                     c->stream));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            for (int64_t i = 0; !dense && i < rows; ++i)
+                memcpy(static_cast<char*>(q.dst) + i * q.size, t.data() + i * q.stride, q.size);
+        }
+        return ISPH_OK;
     }
     // rows of a chunk: columns begin at multiples of 64 rows
     const int64_t most = (int64_t)(SLOT_BYTES / bytes) & ~int64_t(63);
