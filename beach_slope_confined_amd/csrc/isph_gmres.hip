@@ -69,19 +69,30 @@ struct GmMat {
     const double* val;
 };
 
-// K block sums in the tree of block_sum (wave butterfly, (w0+w1)+(w2+w3))
-template <int K>
-__device__ __forceinline__ void block_sum_k(double (&v)[K]) {
-    __shared__ double red[K][4];
+// Eight wave sums in the tree of wave_sum (butterfly, xor 1 to 32); lane l gets
+// that of v[l & 7].  A butterfly leaves the sum of a pair in both its lanes, so
+// in the first three steps each lane adds for half of the values only: 62
+// instructions for 160 (a column 68 -> 66 us at 93k rows).
+__device__ __forceinline__ double wave_sums8(const double (&v)[8]) {
+    const int lane = threadIdx.x & 63;
+    double a[4], b[2];
 #pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = wave_sum(v[k]);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0)
+    for (int p = 0; p < 4; ++p) {
+        const double keep = lane & 1 ? v[2 * p + 1] : v[2 * p];
+        const double send = lane & 1 ? v[2 * p] : v[2 * p + 1];
+        a[p] = keep + lane_move<0xB1>(send);  // quad_perm 1,0,3,2
+    }
 #pragma unroll
-        for (int k = 0; k < K; ++k) red[k][threadIdx.x >> 6] = v[k];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = (red[k][0] + red[k][1]) + (red[k][2] + red[k][3]);
+    for (int p = 0; p < 2; ++p) {
+        const double keep = lane & 2 ? a[2 * p + 1] : a[2 * p];
+        const double send = lane & 2 ? a[2 * p] : a[2 * p + 1];
+        b[p] = keep + lane_move<0x4E>(send);  // quad_perm 2,3,0,1
+    }
+    const double keep = lane & 4 ? b[1] : b[0], send = lane & 4 ? b[0] : b[1];
+    double t = keep + __shfl_xor(send, 4, 64);
+    t = t + lane_move<0x128>(t);  // row_ror 8
+    t = t + __shfl_xor(t, 16, 64);
+    return t + __shfl_xor(t, 32, 64);
 }
 
 // Partials (v_i, w) for i <= j into part[i * nbp + lb]; rows past n add 0.
@@ -91,8 +102,10 @@ __device__ __forceinline__ void block_sum_k(double (&v)[K]) {
 // over the chunks in the kernels that make w and u (one block reduction between
 // a chunk's loads and the next's) those took 38.5 and 38 us at 86k rows, mean
 // of 150 columns; they take 7.7 and 9.9 now and this kernel 9.6 for each.  A
-// column in all: 120 -> 68 us at 93k rows, 243 -> 160 at 319k, 651 -> 501 at
+// column in all: 120 -> 66 us at 93k rows, 243 -> 157 at 319k, 651 -> 498 at
 // 1.01M (whole step over its 150 columns), where the basis comes from HBM.
+// (The second dots together with the subtraction, 64 rows of the basis in LDS,
+// read it once less but leave too few waves to load it: 69, 172 and 529 us.)
 __global__ void __launch_bounds__(BLOCK) k_gm_dots(int n, int j, const double* __restrict__ V,
                                                    size_t cap, const double* __restrict__ w,
                                                    const GmState* st, double* __restrict__ part) {
@@ -108,11 +121,15 @@ __global__ void __launch_bounds__(BLOCK) k_gm_dots(int n, int j, const double* _
     if (done) return;
 #pragma unroll
     for (int k = 0; k < GM_CHUNK; ++k) v[k] = (valid && i0 + k <= j) ? v[k] * wr : 0.0;
-    block_sum_k<GM_CHUNK>(v);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int k = 0; k < GM_CHUNK; ++k)
-            if (i0 + k <= j) part[(size_t)(i0 + k) * gridDim.x + lb] = v[k];
+    __shared__ double red[GM_CHUNK][4];
+    const double t = wave_sums8(v);
+    const int k = threadIdx.x & 63;
+    if (k < GM_CHUNK) red[k][threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x < GM_CHUNK && i0 + (int)threadIdx.x <= j) {  // block_sum's tree
+        const double* q = red[threadIdx.x];
+        part[(size_t)(i0 + threadIdx.x) * gridDim.x + lb] = (q[0] + q[1]) + (q[2] + q[3]);
+    }
 }
 
 // x - h_0 v_0 - h_1 v_1 - ... - h_j v_j at row r, subtracted in order; the
