@@ -453,7 +453,8 @@ class IsphSim(Sim):
         self._check(self._lib.isph_set_progress(self._h, cb, None), "set_progress")
 
     def profile_enable(self, stride=1):
-        """Time every `stride`-th SpMV launch with HIP events (0: off)."""
+        """Time every `stride`-th SpMV launch with HIP events (0: off); while
+        on, BiCGSTAB runs kernel by kernel instead of in one launch."""
         self._check(self._lib.isph_profile_enable(self._h, int(stride)), "profile_enable")
 
     def kernel_time(self, kernel):

@@ -21,7 +21,7 @@ struct CopyTable {
     int first[COPY_MAX];      // first block of an array; past the last one, the number of blocks
 };
 
-__global__ void __launch_bounds__(BLOCK) k_copy(CopyTable t) {
+__global__ void __launch_bounds__(BLOCK) k_copy_arrays(CopyTable t) {
     int a = 0;
 #pragma unroll
     for (int k = 1; k < COPY_MAX; ++k)
@@ -67,7 +67,7 @@ int copy_arrays(isph_ctx* c, const ArrayCopy* a, int n) {
             t.first[k] = (int)blocks;
             blocks += (int64_t)((b + COPY_PIECE - 1) / COPY_PIECE);
         }
-        if (blocks > 0) k_copy<<<(unsigned)blocks, BLOCK, 0, c->stream>>>(t);
+        if (blocks > 0) k_copy_arrays<<<(unsigned)blocks, BLOCK, 0, c->stream>>>(t);
     }
     HIPCHK(c, hipGetLastError());
     return ISPH_OK;

@@ -1723,22 +1723,23 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
     double res = h.nr;            // residual norm now
     double fell = 0.0, took = 0.0;  // log of the residual's fall so far, and its iterations
     for (;;) {
-        // A batch is the iterations that the segment (to the next reliable
-        // update, or to the tolerance) is expected to take at the mean rate so
-        // far, and the update behind them.  An iteration too many costs its
-        // launches, which do nothing (35 us), one too few a wait of the host
-        // (25 us); batches of 8, 4 and 2 by the residual alone launched 22
-        // iterations for 15 at 2.5k rows and waited 9 times, 134 us a needed
-        // iteration where a kernel chain is 60.
+        // A batch is what the segment (to the next reliable update, or to the
+        // tolerance) is expected to take at the mean rate so far, three quarters
+        // of it while it is long, as the rate mostly improves, and the update
+        // behind them.  An iteration too many costs its launches, which do
+        // nothing (35 us), one too few a wait of the host (25 us).  Batches of
+        // 8, 4 and 2 by the residual alone launched 22 iterations for 15 at
+        // 2.5k rows and waited 9 times, 134 us a needed iteration where a kernel
+        // chain is 60; the whole expectation launched 34 for 24 at 1.06M rows.
         const double target = std::max(ctl.tol * h.nb, ctl.delta * h.rupd);
         const double rate = fell > 0.0 ? fell / took : MG_RATE0;
         const double left = res > target ? std::log(res / target) / rate : 0.0;
         const int most = took > 0.0 ? MG_BATCH : MG_BATCH0;
-        const int batch = left < (double)most ? std::max(1, (int)std::ceil(left - 0.25)) : most;
+        const double take = left > 3.0 ? 0.75 * left : left - 0.25;
+        const int batch = take < (double)most ? std::max(1, (int)std::ceil(take)) : most;
         const int before = h.total;
         mg_iterations<T, TI>(c, sys, nbr, ctl, first, batch);
-        const bool tail = batch >= left - 0.25;
-        if (tail) update();
+        update();
         HIPCHK(c, hipGetLastError());
         const int nupd = h.nupd;
         if ((rc = read_sc(c))) return rc;

@@ -1,4 +1,7 @@
-// isph_solver.hip -- BiCGSTAB for the Jacobi-scaled PPE on gfx950.
+// isph_solver.hip -- BiCGSTAB for the Jacobi-scaled PPE on gfx950, a launch a
+// step.  The solves that run in one launch (isph_resident.hip, up to 261k rows;
+// isph_streamed.hip, up to 1.31M) do the same arithmetic; these kernels take
+// the rest: more rows, int32 columns, rows that lie too far apart, timed runs.
 //
 // Recurrences of the reference's bicgstab (solver.f90:162-213, van der
 // Vorst 1992).  One iteration is three row kernels, each followed by a

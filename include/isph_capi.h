@@ -389,7 +389,9 @@ int isph_restore(isph_ctx* ctx, int32_t slot);
  * isph_get_kernel_time() returns the timed launches and their total
  * milliseconds since the last enable.  kernel: 0 = FP64 step-1 SpMV
  * (p update, v = A p), 1 = FP64 step-2 SpMV (s, t = A s), 2 and 3 = the
- * same for the mixed-precision flavours, 4 = scalart. */
+ * same for the mixed-precision flavours, 4 = scalart.  While it is on the
+ * BiCGSTAB solves run kernel by kernel, with the same bits, instead of in the
+ * one launch that they take where the system fits. */
 int isph_profile_enable(isph_ctx* ctx, int32_t enable);
 /* Progress of the long calls: fn(user, what, done, total) is called on the
  * calling thread after each checkpoint segment of isph_adjoint_forward
