@@ -284,13 +284,20 @@ __global__ void __launch_bounds__(ST_THREADS) k_bicg_streamed(KrylovArgs<TV, TX,
         halo[h] = w.x;
         win[place(h)] = w.y;
     }
-    TX* vout = a.si;  // the launched kernels' s and t vectors carry v and t
+    // The launched kernels' s, p and t vectors carry v and t.  Blocks read each
+    // other's t for the last time before they publish their part of the next
+    // iteration's first sum, which its owner collects before it stores t again.
+    // v is read up to the end of the BETA exchange, after the reader's part of
+    // that sum has gone out, so its owner may be at the next v by then: v
+    // alternates between two arrays, and is stored to one of them again after
+    // the next iteration's BETA sum, to which every reader has added since.
     TX* tout = a.mm2;
     coef = sc->betas;
     bool ok = true;
     TX alpha = (TX)0, om = (TX)0;
     for (int it = 0; it < maxiter; ++it) {
         const bool fst = first && it == 0;
+        TX* vout = it & 1 ? a.p : a.si;
         // opaque, so that the rows' addresses are formed where they are used:
         // kept across the iteration they do not fit the registers
         int t = threadIdx.x;
