@@ -153,6 +153,7 @@ def declare(lib, prefix):
 
 
 _LIB = None
+SOLVE_FORMS = ("resident", "streamed", "launched", "refused", "lost")  # ISPH_FORM_*
 
 
 def load_library(path=LIB_PATH):
@@ -173,6 +174,7 @@ def load_library(path=LIB_PATH):
             ("profile_enable", [ctypes.c_void_p, ctypes.c_int32], ctypes.c_int),
             ("get_kernel_time", [ctypes.c_void_p, ctypes.c_int32,
                                  ctypes.POINTER(ctypes.c_int64), _c_dp], ctypes.c_int),
+            ("get_solve_forms", [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64)], ctypes.c_int),
             ("copy_bench", [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, _c_dp], ctypes.c_int),
             ("checkpoint", [ctypes.c_void_p, ctypes.c_int32], ctypes.c_int),
             ("restore", [ctypes.c_void_p, ctypes.c_int32], ctypes.c_int),
@@ -463,6 +465,16 @@ class IsphSim(Sim):
         self._check(self._lib.isph_get_kernel_time(self._h, kernel, ctypes.byref(n),
                                                    ctypes.byref(ms)), "get_kernel_time")
         return n.value, ms.value
+
+    def solve_forms(self):
+        """How the BiCGSTAB solves have run so far, counted by form: one
+        launch with the matrix on the chip ("resident") or from memory
+        ("streamed"), kernel by kernel ("launched"), launches whose blocks
+        could not hold their rows ("refused") and those that the driver
+        refused or that waited in vain ("lost")."""
+        k = (ctypes.c_int64 * len(SOLVE_FORMS))()
+        self._check(self._lib.isph_get_solve_forms(self._h, k), "get_solve_forms")
+        return dict(zip(SOLVE_FORMS, k))
 
     def copy_bench(self, nbytes, reps):
         ms = ctypes.c_double()

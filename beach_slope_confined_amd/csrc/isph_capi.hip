@@ -477,6 +477,7 @@ int iterate(isph_ctx* c, const KrylovArgs<TV, TX, TI>& a, const SolveCtl& ctl, b
             if (resident && c->sc_host->done) return ISPH_OK;
         }
     }
+    c->forms[ISPH_FORM_LAUNCHED] += 1;
     for (;;) {
         const int before = c->sc_host->total;
         int batch = 8;
@@ -1343,6 +1344,12 @@ int isph_get_kernel_time(isph_ctx* c, int32_t kernel, int64_t* launches, double*
     if (!c || kernel < 0 || kernel >= PROF_SLOTS) return ISPH_E_ARG;
     if (launches) *launches = c->prof.launches[kernel];
     if (total_ms) *total_ms = c->prof.total_ms[kernel];
+    return ISPH_OK;
+}
+
+int isph_get_solve_forms(isph_ctx* c, int64_t* counts) {
+    if (!c || !counts) return ISPH_E_ARG;
+    for (int k = 0; k < ISPH_FORMS; ++k) counts[k] = c->forms[k];
     return ISPH_OK;
 }
 

@@ -26,6 +26,7 @@ int grid_launch(isph_ctx* c, const void* kern, int blocks, int threads, void** a
         // is refused, and its contexts keep to the launched kernels.
         (void)hipGetLastError();
         c->cooperative = false;
+        c->forms[ISPH_FORM_LOST] += 1;
         return ISPH_OK;
     }
     uint32_t word[2] = {0, 0};
@@ -36,11 +37,15 @@ int grid_launch(isph_ctx* c, const void* kern, int blocks, int threads, void** a
         // has written its part back, the launched kernels carry on from the
         // state the launch began with, from now on.
         c->cooperative = false;
+        c->forms[ISPH_FORM_LOST] += 1;
         HIPCHK(c, hipMemsetAsync(c->err, 0, sizeof(uint32_t), c->stream));
         if (word[1] & GS_WRITTEN) return fail(c, ISPH_E_HIP, "a resident solve lost a block");
         return ISPH_OK;
     }
-    if (word[1] & GS_REFUSED) return ISPH_OK;
+    if (word[1] & GS_REFUSED) {
+        c->forms[ISPH_FORM_REFUSED] += 1;
+        return ISPH_OK;
+    }
     ran = true;
     return ISPH_OK;
 }

@@ -90,6 +90,7 @@ struct isph_ctx {
     int device = 0, cus = 0;       // GPU of the context, its compute units
     bool cooperative = false;      // it takes cooperative launches
     unsigned long long* gs_words = nullptr;  // exchange words of the resident solves
+    int64_t forms[ISPH_FORMS] = {};          // isph_get_solve_forms
     double2* pos_nb = nullptr;     // positions at the last neighbour search
     double* cdiff = nullptr;       // salinity rate of the last scalart
     double4* salt_coef = nullptr;  // per particle (Dx, Dy, Dm + nut/ts, nut)

@@ -624,7 +624,10 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
     int f = first, m = maxiter, l = kl;
     void* args[] = {&a, &gs, &sc, &t, &h, &f, &m, &l};
     if (int rc = grid_launch(c, (const void*)kern, blocks, R, args, lds, GS_MAXB, ran)) return rc;
-    if (ran) first = false;
+    if (ran) {
+        first = false;
+        c->forms[ISPH_FORM_RESIDENT] += 1;
+    }
     return ISPH_OK;
 }
 

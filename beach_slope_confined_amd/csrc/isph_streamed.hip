@@ -471,7 +471,10 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
     if (int rc = grid_launch(c, (const void*)k_bicg_streamed<TV, TX, J>, GS_MAXB, ST_THREADS, args,
                              RESIDENT_LDS, parts + ST_COPIES * ST_GROUPS, ran))
         return rc;
-    if (ran) first = false;
+    if (ran) {
+        first = false;
+        c->forms[ISPH_FORM_STREAMED] += 1;
+    }
     return ISPH_OK;
 }
 

@@ -393,6 +393,20 @@ int isph_restore(isph_ctx* ctx, int32_t slot);
  * BiCGSTAB solves run kernel by kernel, with the same bits, instead of in the
  * one launch that they take where the system fits. */
 int isph_profile_enable(isph_ctx* ctx, int32_t enable);
+/* How the BiCGSTAB solves of this context have run, counted since its creation:
+ * launches that iterated in one cooperative kernel with the matrix on the chip
+ * or streamed from memory, solves (or their parts between two reliable updates)
+ * that iterated kernel by kernel, cooperative launches that did nothing because
+ * a block could not hold the rows that its rows refer to, and those that the
+ * driver refused or that waited in vain for a block.  All of them give the same
+ * bits.  The multigrid and GMRES solves are not counted. */
+#define ISPH_FORM_RESIDENT 0
+#define ISPH_FORM_STREAMED 1
+#define ISPH_FORM_LAUNCHED 2
+#define ISPH_FORM_REFUSED  3
+#define ISPH_FORM_LOST     4
+#define ISPH_FORMS         5
+int isph_get_solve_forms(isph_ctx* ctx, int64_t counts[ISPH_FORMS]);
 /* Progress of the long calls: fn(user, what, done, total) is called on the
  * calling thread after each checkpoint segment of isph_adjoint_forward
  * (what = "adjoint_forward") and of isph_adjoint_backward
