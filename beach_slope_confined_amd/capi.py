@@ -175,6 +175,7 @@ def load_library(path=LIB_PATH):
             ("get_kernel_time", [ctypes.c_void_p, ctypes.c_int32,
                                  ctypes.POINTER(ctypes.c_int64), _c_dp], ctypes.c_int),
             ("get_solve_forms", [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64)], ctypes.c_int),
+            ("lose_solves", [ctypes.c_void_p, ctypes.c_int32], ctypes.c_int),
             ("copy_bench", [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, _c_dp], ctypes.c_int),
             ("checkpoint", [ctypes.c_void_p, ctypes.c_int32], ctypes.c_int),
             ("restore", [ctypes.c_void_p, ctypes.c_int32], ctypes.c_int),
@@ -475,6 +476,10 @@ class IsphSim(Sim):
         k = (ctypes.c_int64 * len(SOLVE_FORMS))()
         self._check(self._lib.isph_get_solve_forms(self._h, k), "get_solve_forms")
         return dict(zip(SOLVE_FORMS, k))
+
+    def lose_solves(self, n):
+        """The next n cooperative launches end as if they had waited in vain."""
+        self._check(self._lib.isph_lose_solves(self._h, int(n)), "lose_solves")
 
     def copy_bench(self, nbytes, reps):
         ms = ctypes.c_double()

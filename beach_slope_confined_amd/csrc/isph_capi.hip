@@ -124,6 +124,14 @@ int take_errors(isph_ctx* c) {
     return fail(c, ISPH_E_HIP, "unknown device error");
 }
 
+__global__ void k_clear_bits(uint32_t* word, uint32_t bits) { *word &= ~bits; }
+
+int clear_errors(isph_ctx* c, uint32_t bits) {
+    k_clear_bits<<<1, 1, 0, c->stream>>>(c->err, bits);
+    HIPCHK(c, hipGetLastError());
+    return ISPH_OK;
+}
+
 int sync_check(isph_ctx* c) {
     HIPCHK(c, hipGetLastError());
     return take_errors(c);
@@ -1344,6 +1352,12 @@ int isph_get_kernel_time(isph_ctx* c, int32_t kernel, int64_t* launches, double*
     if (!c || kernel < 0 || kernel >= PROF_SLOTS) return ISPH_E_ARG;
     if (launches) *launches = c->prof.launches[kernel];
     if (total_ms) *total_ms = c->prof.total_ms[kernel];
+    return ISPH_OK;
+}
+
+int isph_lose_solves(isph_ctx* c, int32_t n) {
+    if (!c || n < 0) return ISPH_E_ARG;
+    c->lose = n;
     return ISPH_OK;
 }
 

@@ -89,6 +89,7 @@ struct isph_ctx {
     uint32_t* err = nullptr;       // error bits; [1]: a resident solve's GS_* state
     int device = 0, cus = 0;       // GPU of the context, its compute units
     bool cooperative = false;      // it takes cooperative launches
+    int lose = 0;                  // cooperative launches to lose (isph_lose_solves)
     unsigned long long* gs_words = nullptr;  // exchange words of the resident solves
     int64_t forms[ISPH_FORMS] = {};          // isph_get_solve_forms
     double2* pos_nb = nullptr;     // positions at the last neighbour search
@@ -189,6 +190,10 @@ int copy_arrays(isph_ctx* c, const ArrayCopy* a, int n);
 constexpr int STATE_ARRAYS = 19;
 // the copies of the first n rows of state a to b; returns STATE_ARRAYS
 int state_copies(const StateView& a, const StateView& b, int n, ArrayCopy* out);
+
+// takes these bits out of the error word; those that earlier kernels of the
+// step have raised stay for take_errors
+int clear_errors(isph_ctx* c, uint32_t bits);
 
 int alloc_state(isph_ctx* c, StateView& s, size_t cap);
 void free_state(StateView& s);

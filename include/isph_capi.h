@@ -407,6 +407,10 @@ int isph_profile_enable(isph_ctx* ctx, int32_t enable);
 #define ISPH_FORM_LOST     4
 #define ISPH_FORMS         5
 int isph_get_solve_forms(isph_ctx* ctx, int64_t counts[ISPH_FORMS]);
+/* The next n cooperative launches end as if their blocks had waited for each
+ * other in vain, without running: their solves go on kernel by kernel.  For
+ * tests of that. */
+int isph_lose_solves(isph_ctx* ctx, int32_t n);
 /* Progress of the long calls: fn(user, what, done, total) is called on the
  * calling thread after each checkpoint segment of isph_adjoint_forward
  * (what = "adjoint_forward") and of isph_adjoint_backward
