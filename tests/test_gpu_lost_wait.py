@@ -8,6 +8,8 @@ import pytest
 from beach_slope_confined_amd import capi, configs
 from beach_slope_confined_amd.params import PREC_FP64, PREC_MIXED_V64
 
+from parity_util import STAGES, run_stage
+
 pytestmark = pytest.mark.gpu
 
 
@@ -35,17 +37,34 @@ def test_the_launched_kernels_take_over(require_gpu, nside, precision):
         assert np.array_equal(v, out[1][1][k]), k
 
 
+def overflow_before_the_solve(cfg, seed=1):
+    """The configuration with fluid velocities of up to 0.1 dx a step, and its
+    longest neighbour list of the search before the solve, which must be longer
+    than any of the one after: with max_nbr one less, the step's only error is
+    raised before its solve."""
+    p, parts = cfg["params"], {k: v.copy() for k, v in cfg["parts"].items()}
+    fluid = np.flatnonzero(parts["tid"] == 3)
+    v, rng = 0.1 * p.dl / p.dt, np.random.default_rng(seed)
+    parts["vx"][fluid] = rng.uniform(-v, v, len(fluid))
+    parts["vy"][fluid] = rng.uniform(-v, v, len(fluid))
+    cfg = dict(cfg, parts=parts)
+    sim = configs.make_sim(cfg, capi.IsphSim)
+    longest = []
+    for name in STAGES[:STAGES.index("freesurf")]:
+        run_stage(sim, name)
+        if name == "neighbour":
+            longest.append(int(np.diff(sim.get_neighbours()[0]).max()))
+    sim.close()
+    assert longest[0] > longest[1]
+    return dict(cfg, params=p.copy(max_nbr=longest[0] - 1))
+
+
 @pytest.mark.parametrize("lose", [0, 1])
 @pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED_V64])
 def test_pending_errors_are_reported(require_gpu, lose, precision):
     cfg = configs.dam_break(0.01)
     cfg["params"] = cfg["params"].copy(precision=precision, tol=1e-4)
-    sim = configs.make_sim(cfg, capi.IsphSim)
-    sim.neighbour()
-    longest = int(np.diff(sim.get_neighbours()[0]).max())
-    sim.close()
-    cfg["params"] = cfg["params"].copy(max_nbr=longest - 1)
-    sim = configs.make_sim(cfg, capi.IsphSim)
+    sim = configs.make_sim(overflow_before_the_solve(cfg), capi.IsphSim)
     sim.lose_solves(lose)
     with pytest.raises(capi.IsphError, match="ISPH_E_CAPACITY"):
         sim.step(1)
