@@ -566,7 +566,7 @@ int solve_fp64_on(isph_ctx* c, const double* val, const double* rhs, double* x) 
     HIPCHK(c, hipMemcpyAsync(&e, c->err, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (e & ERR_INDEX16) {
-        HIPCHK(c, hipMemsetAsync(c->err, 0, sizeof(uint32_t), c->stream));
+        if (int rc = clear_errors(c, ERR_INDEX16)) return rc;
         c->narrow_idx = false;
         return solve_fp64_t<int>(c, c->nbr, val, rhs, x);
     }
@@ -639,7 +639,8 @@ int solve_mixed(isph_ctx* c) {
     HIPCHK(c, hipMemcpyAsync(&e, c->err, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const bool narrow = !(e & ERR_INDEX16);
-    if (!narrow) HIPCHK(c, hipMemsetAsync(c->err, 0, sizeof(uint32_t), c->stream));
+    if (!narrow)
+        if (int rc = clear_errors(c, ERR_INDEX16)) return rc;
     c->narrow_idx = narrow;
     if (c->prm.precision == ISPH_PREC_MIXED_V64) {
         double* vv[5] = {c->v64[0], c->v64[1], c->v64[2], c->v64[3], c->v64[4]};

@@ -1786,7 +1786,8 @@ int solve_mg_on(isph_ctx* c, const MGSystem& sys) {
     HIPCHK(c, hipMemcpyAsync(&e, c->err, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const bool narrow = !(e & ERR_INDEX16);
-    if (!narrow) HIPCHK(c, hipMemsetAsync(c->err, 0, sizeof(uint32_t), c->stream));
+    if (!narrow)
+        if (int rc = clear_errors(c, ERR_INDEX16)) return rc;
     c->narrow_idx = narrow;
     if (c->prm.precision == ISPH_PREC_FP64_MG)
         return narrow ? solve_mg_t<double, short>(c, sys, c->nbr16)
