@@ -342,7 +342,11 @@ __device__ __forceinline__ void resident_leader(const GridSync& gs, int nw, Solv
         gs_broadcast(gs, e, s.betas, s.done);
         if (s.done) break;
     }
-    if (t == 0) *sc = s;
+    if (t == 0) {
+        // ahead of the vectors, should the workers lose the last broadcast
+        atomicOr(gs.state, GS_WRITTEN);
+        *sc = s;
+    }
 }
 
 // NP > 0: no leader; one wave of every block sums all parts, up to 64 NP, and
