@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -48,13 +49,43 @@ namespace host {
 
 namespace {
 
-// Pinned staging of the process: one slot a thread.  Allocated at the first
-// download, kept while contexts live (10 MB), given back with the last one.
+// Pinned staging of the process: slots that the downloads of all contexts share,
+// a chunk at a time.  Allocated at the first download, kept while contexts live
+// (10 MB), given back with the last one.  Whoever holds a slot waits for nothing
+// but its own chunk, so contexts on other streams and GPUs go on meanwhile.
 constexpr int SLOTS = 8;
 constexpr size_t SLOT_BYTES = 1280 * 1024;
 std::mutex pool_lock;
+std::condition_variable pool_given;
 char* pool = nullptr;
 int pool_users = 0;
+unsigned pool_free = (1u << SLOTS) - 1;
+
+// the pool's memory; null if there is none to be had
+char* pool_memory() {
+    std::lock_guard<std::mutex> g(pool_lock);
+    if (!pool && hipHostMalloc((void**)&pool, SLOTS * SLOT_BYTES, hipHostMallocPortable) != hipSuccess) {
+        pool = nullptr;
+        (void)hipGetLastError();
+    }
+    return pool;
+}
+
+int take_slot() {
+    std::unique_lock<std::mutex> g(pool_lock);
+    pool_given.wait(g, [] { return pool_free != 0; });
+    const int slot = __builtin_ctz(pool_free);
+    pool_free &= ~(1u << slot);
+    return slot;
+}
+
+void give_slot(int slot) {
+    {
+        std::lock_guard<std::mutex> g(pool_lock);
+        pool_free |= 1u << slot;
+    }
+    pool_given.notify_one();
+}
 
 }  // namespace
 
@@ -75,12 +106,9 @@ int download(isph_ctx* c, int64_t rows, const Column* cols, int ncol) {
     if (rows <= 0 || ncol <= 0) return ISPH_OK;
     size_t bytes = 0;  // of a row
     for (int k = 0; k < ncol; ++k) bytes += cols[k].size;
-    std::lock_guard<std::mutex> g(pool_lock);
-    if (!pool && hipHostMalloc((void**)&pool, SLOTS * SLOT_BYTES, hipHostMallocPortable) != hipSuccess) {
-        pool = nullptr;
-        (void)hipGetLastError();
-    }
-    if (!pool) {  // no pinned memory: through the runtime's own staging
+    HIPCHK(c, hipStreamSynchronize(c->stream));  // before a slot is held
+    char* const mem = pool_memory();
+    if (!mem) {  // no pinned memory: through the runtime's own staging
         std::vector<char> t;
         for (int k = 0; k < ncol; ++k) {
             const Column& q = cols[k];
@@ -111,24 +139,26 @@ int download(isph_ctx* c, int64_t rows, const Column* cols, int ncol) {
     }
     std::atomic<int64_t> next{0};
     std::atomic<int> status{hipSuccess};
-    auto work = [&](int slot) {
-        char* buf = pool + (size_t)slot * SLOT_BYTES;
+    auto work = [&](int thread) {
         hipEvent_t ev = nullptr;
         // a thread of our own starts on device 0; the caller's is the caller's
-        hipError_t e = slot ? hipSetDevice(c->device) : hipSuccess;
+        hipError_t e = thread ? hipSetDevice(c->device) : hipSuccess;
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
         while (e == hipSuccess && status.load() == hipSuccess) {
             const int64_t r0 = per * next.fetch_add(1);
             if (r0 >= rows) break;
             const int m = (int)std::min<int64_t>(per, rows - r0);
+            const int slot = take_slot();
+            char* buf = mem + (size_t)slot * SLOT_BYTES;
             k_pack<<<nblk(m), BLOCK, 0, c->stream>>>(r0, m, pc, buf);
             e = hipGetLastError();
             if (e == hipSuccess) e = hipEventRecord(ev, c->stream);
             if (e == hipSuccess) e = hipEventSynchronize(ev);
-            if (e != hipSuccess) break;
-            for (int k = 0; k < ncol; ++k)
+            for (int k = 0; e == hipSuccess && k < ncol; ++k)
                 memcpy(static_cast<char*>(cols[k].dst) + (size_t)r0 * cols[k].size,
                        buf + pc.at[k], (size_t)m * cols[k].size);
+            if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);  // it may be written still
+            give_slot(slot);
         }
         if (ev) (void)hipEventDestroy(ev);
         if (e != hipSuccess) status.store(e);
