@@ -87,6 +87,27 @@ void give_slot(int slot) {
     pool_given.notify_one();
 }
 
+// The calling thread works on a device for as long as this lives: a launch and
+// an event belong to the current device, a copy on a stream did not need it.
+class OnDevice {
+public:
+    explicit OnDevice(int device) {
+        status = hipGetDevice(&before);
+        if (status == hipSuccess && before != device) {
+            status = hipSetDevice(device);
+            moved = status == hipSuccess;
+        }
+    }
+    ~OnDevice() {
+        if (moved) (void)hipSetDevice(before);
+    }
+    hipError_t status;
+
+private:
+    int before = 0;
+    bool moved = false;
+};
+
 }  // namespace
 
 void transfer_attach() {
@@ -106,6 +127,8 @@ int download(isph_ctx* c, int64_t rows, const Column* cols, int ncol) {
     if (rows <= 0 || ncol <= 0) return ISPH_OK;
     size_t bytes = 0;  // of a row
     for (int k = 0; k < ncol; ++k) bytes += cols[k].size;
+    const OnDevice there(c->device);
+    HIPCHK(c, there.status);
     HIPCHK(c, hipStreamSynchronize(c->stream));  // before a slot is held
     char* const mem = pool_memory();
     if (!mem) {  // no pinned memory: through the runtime's own staging
@@ -141,7 +164,7 @@ int download(isph_ctx* c, int64_t rows, const Column* cols, int ncol) {
     std::atomic<int> status{hipSuccess};
     auto work = [&](int thread) {
         hipEvent_t ev = nullptr;
-        // a thread of our own starts on device 0; the caller's is the caller's
+        // a thread of our own starts on device 0
         hipError_t e = thread ? hipSetDevice(c->device) : hipSuccess;
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
         while (e == hipSuccess && status.load() == hipSuccess) {

@@ -30,7 +30,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["busy", "busy_unpinned", "crowd"])
+@pytest.mark.parametrize("scenario", ["busy", "busy_unpinned", "crowd", "device"])
 def test_downloads(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -172,6 +172,16 @@ static void crowd(int rows) {
     for (auto& t : th) t.join();
 }
 
+// The calling thread's current device is another than the context's, and stays so.
+static void device(int rows) {
+    Particles p(rows, 1, 5);
+    CHECK(hipSetDevice(2) == hipSuccess);
+    CHECK(p.get() == ISPH_OK && p.right());
+    int now = -1;
+    CHECK(hipGetDevice(&now) == hipSuccess && now == 2);
+    transfer_detach();
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     for (int rows : {1, 65, 200000, 700001}) {
@@ -181,6 +191,7 @@ int main(int argc, char** argv) {
             busy(rows);
         }
         if (what == "crowd") crowd(rows);
+        if (what == "device") device(rows);
     }
     return 0;
 }
