@@ -1,4 +1,6 @@
 // isph_gridsync.hip -- launching grids whose blocks wait for each other.
+#include <algorithm>
+
 #include "isph_gridsync.h"
 #include "isph_host.h"
 
@@ -30,12 +32,16 @@ int grid_launch(isph_ctx* c, const void* kern, int blocks, int threads, void** a
         e = hipLaunchCooperativeKernel(kern, dim3(blocks), dim3(threads), args, (unsigned)lds,
                                        c->stream);
     }
+    auto lost = [&] {
+        c->hold = c->hold_next;
+        c->hold_next = std::min(2 * c->hold_next, HOLD_MOST);
+        c->forms[ISPH_FORM_LOST] += 1;
+    };
     if (e != hipSuccess) {
         // One process at a time holds a GPU's cooperative queue; a second one
-        // is refused, and its contexts keep to the launched kernels.
+        // is refused, and its contexts keep to the launched kernels meanwhile.
         (void)hipGetLastError();
-        c->cooperative = false;
-        c->forms[ISPH_FORM_LOST] += 1;
+        lost();
         return ISPH_OK;
     }
     uint32_t word[2] = {0, 0};
@@ -44,9 +50,8 @@ int grid_launch(isph_ctx* c, const void* kern, int blocks, int threads, void** a
     if (word[0] & ERR_SYNC) {
         // Blocks waited in vain: something else holds their CUs.  Unless one
         // has written its part back, the launched kernels carry on from the
-        // state the launch began with, from now on.
-        c->cooperative = false;
-        c->forms[ISPH_FORM_LOST] += 1;
+        // state the launch began with.
+        lost();
         if (int rc = clear_errors(c, ERR_SYNC)) return rc;
         if (word[1] & GS_WRITTEN) return fail(c, ISPH_E_HIP, "a resident solve lost a block");
         return ISPH_OK;
@@ -55,6 +60,7 @@ int grid_launch(isph_ctx* c, const void* kern, int blocks, int threads, void** a
         c->forms[ISPH_FORM_REFUSED] += 1;
         return ISPH_OK;
     }
+    c->hold_next = HOLD_FIRST;
     ran = true;
     return ISPH_OK;
 }

@@ -55,6 +55,13 @@ struct BufferZone {
 
 #define ISPH_MAX_DEVICES 64  // GPUs per process the library keeps per-device addresses for
 
+// A cooperative launch that the driver refuses (another process holds the queue)
+// or that waits in vain (something else holds its CUs: about a second lost) is
+// not tried again for 64 solves, then twice as many each time, until one runs.
+namespace isph {
+constexpr int HOLD_FIRST = 64, HOLD_MOST = 1 << 16;
+}
+
 struct isph_ctx {
     isph_params prm;
     int32_t cap = 0, cap_soil = 0, n = 0, ns = 0;
@@ -89,6 +96,8 @@ struct isph_ctx {
     uint32_t* err = nullptr;       // error bits; [1]: a resident solve's GS_* state
     int device = 0, cus = 0;       // GPU of the context, its compute units
     bool cooperative = false;      // it takes cooperative launches
+    int hold = 0;                  // solves to run kernel by kernel before the next one,
+    int hold_next = isph::HOLD_FIRST;  // and after the next one that is refused or lost
     int lose = 0;                  // cooperative launches to lose (isph_lose_solves)
     unsigned long long* gs_words = nullptr;  // exchange words of the resident solves
     int64_t forms[ISPH_FORMS] = {};          // isph_get_solve_forms

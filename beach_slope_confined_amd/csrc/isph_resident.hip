@@ -649,6 +649,10 @@ int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const Solv
                      bool& first, int maxiter, bool& ran) {
     ran = false;
     if (!c->cooperative || c->n == 0) return ISPH_OK;
+    if (c->hold > 0) {
+        c->hold -= 1;
+        return ISPH_OK;
+    }
     const int nb = nblk(c->n), most = GS_MAXB - 1;
     if (nb <= 64) return launch<TV, TX, 1, 1>(c, a, ctl, first, maxiter, ran);
     if (nb <= 128) return launch<TV, TX, 2, 1>(c, a, ctl, first, maxiter, ran);

@@ -487,7 +487,7 @@ int streamed_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const Solv
     const int np = nblk(c->n);
     // a block per CU with rows in each; entry counts share a register with
     // the diagonal's position; 32-bit byte offsets into the values
-    if (!c->cooperative || c->cus < GS_MAXB || np < GS_MAXB || np > ST_MAXP * FIN_BLOCK ||
+    if (c->cus < GS_MAXB || np < GS_MAXB || np > ST_MAXP * FIN_BLOCK ||
         c->prm.max_nbr > 0x7fff || (uint64_t)c->prm.max_nbr * a.ld * sizeof(TV) > 0xffffffffull)
         return ISPH_OK;
     const int most = (np + GS_MAXB - 1) / GS_MAXB * BLOCK;  // rows of a block

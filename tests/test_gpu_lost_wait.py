@@ -70,3 +70,24 @@ def test_pending_errors_are_reported(require_gpu, lose, precision):
         sim.step(1)
     assert sim.solve_forms()["lost"] == lose
     sim.close()
+
+
+def test_one_launch_again_after_a_while(require_gpu):
+    """Two lost launches in a row keep 64 and then 128 solves kernel by kernel;
+    the next one runs in one launch again, and one that is lost later counts
+    from 64 anew.  The run's bits are those of one that lost none."""
+    sims = [configs.make_sim(configs.dam_break(0.01), capi.IsphSim) for _ in range(2)]
+    for lose, launched in ((2, (1 + 64) + (1 + 128)), (1, 1 + 64)):
+        before = sims[1].solve_forms()
+        sims[1].lose_solves(lose)
+        for _ in range(launched + 1):
+            for sim in sims:
+                sim.step(1)
+            now = sims[1].solve_forms()
+            if now["resident"] > before["resident"]:
+                break
+        assert now["lost"] - before["lost"] == lose
+        assert now["launched"] - before["launched"] == launched
+    a, b = (sim.get_particles() for sim in sims)
+    for k in a:
+        assert np.array_equal(a[k], b[k]), k
