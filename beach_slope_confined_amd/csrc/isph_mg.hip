@@ -1743,11 +1743,6 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
         HIPCHK(c, hipGetLastError());
         const int nupd = h.nupd;
         if ((rc = read_sc(c))) return rc;
-        if (h.done == DONE_UPDATE) {
-            update();
-            HIPCHK(c, hipGetLastError());
-            if ((rc = read_sc(c))) return rc;
-        }
         if (h.done == DONE_CONVERGED) return ISPH_OK;
         if (h.done == DONE_FAILED) return fail(c, ISPH_E_NOCONV, "multigrid PPE solve did not converge");
         if (h.done != DONE_RUNNING) return fail(c, ISPH_E_STATE, "unexpected solver state");
