@@ -479,20 +479,20 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
 }
 
 // Rows a thread, from the most 256-row blocks that one of 256 blocks gets: 2
-// up to 393k rows, 7 up to 1.31M.
+// up to 393k rows, 7 up to 1.31M.  Called above 261,120 rows, so every block has
+// rows.
 template <class TV, class TX>
 int streamed_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
                      bool& first, int maxiter, bool& ran) {
     ran = false;
     const int np = nblk(c->n);
-    // a block per CU with rows in each; entry counts share a register with
-    // the diagonal's position; 32-bit byte offsets into the values
-    if (c->cus < GS_MAXB || np < GS_MAXB || np > ST_MAXP * FIN_BLOCK ||
-        c->prm.max_nbr > 0x7fff || (uint64_t)c->prm.max_nbr * a.ld * sizeof(TV) > 0xffffffffull)
+    // a block per CU; entry counts share a register with the diagonal's
+    // position; 32-bit byte offsets into the values
+    if (c->cus < GS_MAXB || np > ST_MAXP * FIN_BLOCK || c->prm.max_nbr > 0x7fff ||
+        (uint64_t)c->prm.max_nbr * a.ld * sizeof(TV) > 0xffffffffull)
         return ISPH_OK;
     const int most = (np + GS_MAXB - 1) / GS_MAXB * BLOCK;  // rows of a block
     switch ((most + ST_THREADS - 1) / ST_THREADS) {
-        case 1:
         case 2: return launch<TV, TX, 2>(c, a, ctl, first, maxiter, ran);
         case 3: return launch<TV, TX, 3>(c, a, ctl, first, maxiter, ran);
         case 4: return launch<TV, TX, 4>(c, a, ctl, first, maxiter, ran);
