@@ -14,10 +14,11 @@ shifting, timestep reduction.
 Prints one JSON line.  `value` is fluid particle-steps/s of the FP64 step;
 the mixed-precision PPE step on the same input is reported beside it
 (`mixed`), with its pressure and velocity error against the FP64 step.
-`roofline` is the dominant kernel (a BiCGSTAB SpMV kernel) timed with HIP
-events on the library's stream during the timed steps; `cpu_baseline` is
-the CPU oracle (this repository's C restatement of the reference step,
-OpenMP) on the host cores of the same machine.
+`roofline` is the dominant kernel: the solve's one launch per iteration, and
+beside it the SpMV kernel that is launched in its place while kernels are
+timed (HIP events on the library's stream); `cpu_baseline` is the CPU oracle
+(this repository's C restatement of the reference step, OpenMP) on the host
+cores of the same machine.
 """
 import argparse
 import json
@@ -32,6 +33,8 @@ sys.path.insert(0, ROOT)
 
 METRIC = "ISPH particle-steps/s @1M (FP64 vs mixed-prec PPE); adjoint/forward cost"
 HBM_PEAK_GBS = 8000.0
+STAGES = ("projection", "cellshift", "resetid", "neighbour", "effpor", "eddyvis", "int_vel",
+          "ppe_assemble")  # of a step, up to its solve
 PROFILE_STRIDE = 16  # HIP events around every 16th SpMV launch of the profiled step
 
 
@@ -85,12 +88,25 @@ def model_spmv_bytes(n, nnz_off):
     return 32 * n + 12 * nnz_off
 
 
-def model_step_bytes(n, nnz_off, iters):
-    """Algorithmic bytes of one FP64 step in the same model: per row the
-    fixed stages 1284 + 60 K and per BiCGSTAB iteration 248 + 24 K (two
-    SpMVs, five dots, a norm, three axpys)."""
-    k = nnz_off / n
-    return n * ((1284 + 60 * k) + iters * (248 + 24 * k))
+def iteration_bytes(form, nnz_off, n, val_bytes, idx_bytes):
+    """Algorithmic bytes of one BiCGSTAB iteration with FP64 vectors.
+    Kernel by kernel: 248 + 24 K a row (two SpMVs of 12 K, five dots, a norm,
+    three axpys).  In one launch the row's vectors stay on the chip: rhat is
+    read twice, v and t are written, and read by the blocks that border on
+    the row (48), and the matrix, values and offsets, is read twice (FP32
+    values: and the row sums, 16).  Where it stays on the chip too, v and t
+    are left (32)."""
+    if form == "resident":
+        return 32 * n
+    if form == "streamed":
+        return (48 + (16 if val_bytes == 4 else 0)) * n + 2 * (val_bytes + idx_bytes) * nnz_off
+    return 248 * n + 24 * nnz_off
+
+
+def model_step_bytes(n, nnz_off, iters, per_iteration):
+    """Algorithmic bytes of one FP64 step: per row the fixed stages, 1284 +
+    60 K, and the iterations."""
+    return 1284 * n + 60 * nnz_off + iters * per_iteration
 
 
 def kernel_bytes(kind, nnz_off, n, val_bytes, vec_bytes, idx_bytes=4):
@@ -152,6 +168,20 @@ def run_gpu(cfg, steps, warmup, precision, profile, tol=None, maxit=200000, list
         narrow = bool(len(idx) == 0 or np.abs(idx.astype(np.int64) - rows).max() <= 32767)
         out.update(nnz_off=int(ptr[-1]), n=len(ptr) - 1, idx_bytes=2 if narrow else 4)
     if profile:
+        # the solve alone, in the form that the timed steps give it
+        sim.restore(0)
+        q = sim.scalars()
+        sim.set_scalars(q["umax"], q["dt"], q["t"] + q["dt"])
+        for name in STAGES:
+            getattr(sim, name)()
+        f0 = sim.solve_forms()
+        t0 = time.perf_counter()
+        its, _ = sim.ppe_solve()
+        t1 = time.perf_counter()
+        f1 = sim.solve_forms()
+        ran = {k: f1[k] - f0[k] for k in f1 if f1[k] > f0[k]}
+        out["solve"] = dict(form=max(ran, key=ran.get), launches=sum(ran.values()),
+                            us_per_iteration=1e6 * (t1 - t0) / max(its, 1))
         # the solver's SpMV kernels are timed in one more step: while they are,
         # the solve runs kernel by kernel instead of in one cooperative launch
         sim.restore(0)
@@ -705,7 +735,7 @@ def main():
     value = n_fluid * args.steps / r64["seconds"]
     timed_iters = r64["iters"][args.warmup:]
 
-    # roofline of the dominant kernel (larger total time of the two SpMV kernels)
+    # the SpMV kernel with the larger total time, kernel by kernel
     kt = r64["ktime"]
     dom = max(kt, key=lambda k: kt[k][1])
     launches, tot = kt[dom]
@@ -718,35 +748,53 @@ def main():
     ti = "short" if r64["idx_bytes"] == 2 else "int"
     kname = (f"k_krylov_1t<double, double, {ti}, false>" if dom == "p_spmv"
              else f"k_krylov_2<double, double, {ti}>")
-    roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
+    launched = {"achieved": round(achieved, 1), "unit": "GB/s",
+                "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
                 "kernel": kname, "launches": launches, "avg_us": round(avg_s * 1e6, 2),
                 "bytes_per_launch": nbytes,
                 "bytes_model": "32 + 12K per row, K = %.3f off-diagonal entries per row"
                                % (r64["nnz_off"] / r64["n"]),
                 "own_bytes_per_launch": own,
                 "own_frac": round(own / avg_s / 1e9 / HBM_PEAK_GBS, 4) if launches else None}
+    # the dominant kernel of the timed steps
+    solve = r64["solve"]
+    ib = iteration_bytes(solve["form"], r64["nnz_off"], r64["n"], 8, r64["idx_bytes"])
+    rate = ib / solve["us_per_iteration"] / 1e3
+    roofline = {"bound": "exchanges" if solve["form"] == "resident" else "hbm",
+                "achieved": round(rate, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(rate / HBM_PEAK_GBS, 4), "traffic": None,
+                "kernel": {"resident": "k_bicg_resident", "streamed": "k_bicg_streamed"}.get(
+                    solve["form"], kname),
+                "launches": solve["launches"],
+                "us_per_iteration": round(solve["us_per_iteration"], 2),
+                "bytes_per_iteration": ib,
+                "bytes_model": {"resident": "32 per row: the system stays on the chip",
+                                "streamed": "48 + %dK per row: the matrix twice, partly from "
+                                            "the Infinity Cache" % (2 * (8 + r64["idx_bytes"]))}
+                .get(solve["form"], "248 + 24K per row"),
+                "kernel_by_kernel": launched}
     # attainable streaming bandwidth on this GPU: a 1 GiB copy (read + write)
     try:
         cms = r64["sim"].copy_bench(1 << 30, 10)
         copy_gbs = 2 * (1 << 30) / cms / 1e6
         roofline["copy_GBs"] = round(copy_gbs, 1)
-        roofline["frac_of_copy"] = round(achieved / copy_gbs, 4)
+        roofline["frac_of_copy"] = round(rate / copy_gbs, 4)
+        launched["frac_of_copy"] = round(achieved / copy_gbs, 4)
     except Exception as e:  # reported, not hidden
         roofline["copy_GBs"] = {"error": str(e)}
-    sb = model_step_bytes(r64["n"], r64["nnz_off"], timed_iters[-1])
+    sb = model_step_bytes(r64["n"], r64["nnz_off"], timed_iters[-1], ib)
     step_model = {"bytes_per_step": round(sb), "achieved": round(sb / (ms / 1e3) / 1e9, 1),
                   "unit": "GB/s", "frac": round(sb / (ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
-                  "model": "rows x (1284 + 60K + iterations x (248 + 24K)) bytes"}
+                  "model": "rows x (1284 + 60K) bytes + iterations x %d" % ib}
     pmc = os.path.join(ROOT, "profiles", "bicg_spmv_traffic.json")
     if os.path.exists(pmc):
         with open(pmc) as f:
             d = json.load(f)
-        roofline["traffic"] = d.get(roofline["kernel"], {}).get("hbm_bytes_per_launch")
-        if roofline["traffic"]:
-            roofline["traffic_source"] = ("profiles/bicg_spmv_traffic.json: rocprofv3 --pmc, "
+        launched["traffic"] = d.get(kname, {}).get("hbm_bytes_per_launch")
+        if launched["traffic"]:
+            launched["traffic_source"] = ("profiles/bicg_spmv_traffic.json: rocprofv3 --pmc, "
                                           "read bytes by request size, WRITE_SIZE")
-            roofline["traffic_over_model"] = round(roofline["traffic"] / nbytes, 3)
+            launched["traffic_over_model"] = round(launched["traffic"] / nbytes, 3)
 
     line = {
         "metric": METRIC, "value": round(value, 1), "unit": "particle-steps/s", "n_gpus": 1,
@@ -788,6 +836,11 @@ def main():
             avgm = tm / max(lm, 1) / 1e3
             # FP32 values, 16-bit column offsets, vectors of vb bytes
             bm = kernel_bytes(domm, rmx["nnz_off"], rmx["n"], 4, vb, rmx["idx_bytes"])
+            sol = dict(rmx["solve"], us_per_iteration=round(rmx["solve"]["us_per_iteration"], 2))
+            if vb == 8:
+                sol["achieved_GBs"] = round(
+                    iteration_bytes(sol["form"], rmx["nnz_off"], rmx["n"], 4, rmx["idx_bytes"])
+                    / rmx["solve"]["us_per_iteration"] / 1e3, 1)
             line[key] = {
                 "value": round(vmx, 1), "ms_per_step": round(1e3 * rmx["seconds"] / args.steps, 3),
                 "speedup_vs_fp64": round(vmx / value, 3),
@@ -795,11 +848,13 @@ def main():
                 "iters_per_step": rmx["iters"][args.warmup:], "reliable_updates": rmx["outer"],
                 "relres": rmx["relres"], "pressure_err_vs_fp64": perr,
                 "velocity_err_vs_fp64": verr,
-                "dominant_kernel": {"kernel": f"k_krylov_{'1t' if domm == 'p_spmv' else 2}<float, "
-                                              f"{'double' if vb == 8 else 'float'}, "
-                                              f"{'short' if rmx['idx_bytes'] == 2 else 'int'}>",
-                                    "avg_us": round(avgm * 1e6, 2),
-                                    "achieved_GBs": round(bm / avgm / 1e9, 1) if lm else None},
+                "solve": sol,
+                "kernel_by_kernel": {
+                    "kernel": f"k_krylov_{'1t' if domm == 'p_spmv' else 2}<float, "
+                              f"{'double' if vb == 8 else 'float'}, "
+                              f"{'short' if rmx['idx_bytes'] == 2 else 'int'}>",
+                    "avg_us": round(avgm * 1e6, 2),
+                    "achieved_GBs": round(bm / avgm / 1e9, 1) if lm else None},
             }
             rmx["sim"].close()
 
