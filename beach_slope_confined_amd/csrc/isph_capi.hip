@@ -465,8 +465,9 @@ KrylovArgs<TV, TX, TI> krylov_args(isph_ctx* c, const TI* nbr, const TV* val, TX
     return a;
 }
 
-// iterations per launch of a resident solve: a launch ends within tens of
-// milliseconds, and the next one carries on from the state it left
+// iterations per launch of a resident solve, after which the next launch carries
+// on from the state it left: a launch ends within 25 ms at 2.5k rows, 80 ms at
+// 255k, 0.34 s at 1.06M
 constexpr int RESIDENT_ITERS = 4096;
 
 // BiCGSTAB iterations in batches until the device sets sc->done; the host

@@ -238,7 +238,8 @@ int solve_fp64_on(isph_ctx* c, const double* val, const double* rhs, double* x);
 // Up to maxiter BiCGSTAB iterations in one cooperative launch
 // (isph_resident.hip); on return sc_host holds the state and `first` is
 // cleared.  `ran` is false, and nothing has changed, when the system is too
-// large, its rows reach too far, or the GPU cannot hold the grid.  (Offsets
+// large, its rows reach too far, the GPU cannot hold the grid, or an earlier
+// launch was lost (isph_ctx::hold).  (Offsets
 // that do not fit 16 bits reach too far.)
 constexpr size_t RESIDENT_LDS = 152 * 1024;  // of a CU's 160 KB, beside the static shared memory
 template <class TV, class TX>

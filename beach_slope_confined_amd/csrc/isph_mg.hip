@@ -1730,7 +1730,11 @@ static int solve_mg_body(isph_ctx* c, const MGSystem& sys, const TI* nbr) {
         // nothing (35 us), one too few a wait of the host (25 us).  Batches of
         // 8, 4 and 2 by the residual alone launched 22 iterations for 15 at
         // 2.5k rows and waited 9 times, 134 us a needed iteration where a kernel
-        // chain is 60; the whole expectation launched 34 for 24 at 1.06M rows.
+        // chain is 60; the whole expectation launched 34 for 24 at 1.06M rows,
+        // three quarters 28.  Against the batches by the residual 2.5k rows gain
+        // 1.18x by the rate and 1.2% more by the three quarters, 1.06M rows -0.3
+        // and 2.6%, 133k forward and back 1 and 0.2%, 4.26M 0.8 and -0.1% (296
+        // launched for 282).
         const double target = std::max(ctl.tol * h.nb, ctl.delta * h.rupd);
         const double rate = fell > 0.0 ? fell / took : MG_RATE0;
         const double left = res > target ? std::log(res / target) / rate : 0.0;

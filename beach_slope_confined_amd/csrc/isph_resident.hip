@@ -1,7 +1,7 @@
 // isph_resident.hip -- BiCGSTAB iterations of systems that fit on the chip.
 //
 // An iteration of the launched kernels (isph_solver.hip) is six dependent
-// launches, 29 us at 2.5k rows and 32 us at 87k, whatever the work.  Here one
+// launches, 24 us at 2.5k rows and 27 us at 87k, whatever the work.  Here one
 // cooperative launch runs thousands of iterations.  A block owns R = 256 G
 // consecutive rows, one per thread.  The row's matrix entries are copied to
 // LDS once; the row's vector entries stay in registers.  The rows outside the
@@ -29,9 +29,9 @@
 // What bounds it: the chain of three exchanges (1.3 us each without a leader,
 // 2.3 with one: the words' way, the sums on either side), then two products
 // (0.5 us), and with a leader the halo reads (0.4 us) and the wait for the
-// stores.  Measured per iteration, launched kernels and here: 29 and 6.9 us at
-// 2.5k rows, 30 and 7.9 us at 36.6k, 32 and 9.7 us at 86k, 44 and 19 us at
-// 255k.  Values and places in LDS instead of registers, with the diagonal
+// stores.  Measured per iteration of the solve, launched kernels and here: 24.6
+// and 6.1 us at 2.5k rows, 23.4 and 7.7 us at 36.6k, 27 and 9.7 us at 87k, 40
+// and 19 us at 255k.  Values and places in LDS instead of registers, with the diagonal
 // tested at every entry, made a product 1.3 us.
 //
 // The arithmetic is the launched kernels', term for term: the same row sums,
@@ -638,12 +638,13 @@ static int launch(isph_ctx* c, const KrylovArgs<TV, TX, short>& ka, const SolveC
 // Rows per block, 256 G, and whether a leader serves the exchanges.  Up to 192
 // blocks do without (NP parts a lane): the words' round trip saved is more than
 // every block's reading of every part, and so fewer, larger blocks are better
-// from 64 on.  Measured with blocks of 256 and of 512 rows: 6.9 and 6.95 us an
-// iteration at 11k rows, 7.8 / 7.0 at 17.7k, 9.1 / 7.9 at 36.6k, 9.7 / 8.1 at
-// 47k; with and without a leader 11.6 / 8.2 at 59k, 10.8 / 9.4 at 72.5k, 10.9 /
-// 9.7 at 86k, but 11.5 / 13.4 at 103k.  Beyond 98k rows a leader, and beyond
-// 130,560 blocks of 1024 rows, as few as let the grid hold the system with one
-// worker per CU and a CU for the leader, up to 261,120.
+// from 64 on.  A whole step over its iterations (0 to 0.8 us above the solve
+// alone) with blocks of 256 and of 512 rows: 6.9 and 6.95 us an iteration at
+// 11k rows, 7.8 / 7.0 at 17.7k, 9.1 / 7.9 at 36.6k, 9.7 / 8.1 at 47k; with and
+// without a leader 11.6 / 8.2 at 59k, 10.8 / 9.4 at 72.5k, 10.9 / 9.7 at 86k,
+// but 11.5 / 13.4 at 103k.  Beyond 98k rows a leader, and beyond 130,560 blocks
+// of 1024 rows, as few as let the grid hold the system with one worker per CU
+// and a CU for the leader, up to 261,120.
 template <class TV, class TX>
 int resident_iterate(isph_ctx* c, const KrylovArgs<TV, TX, short>& a, const SolveCtl& ctl,
                      bool& first, int maxiter, bool& ran) {

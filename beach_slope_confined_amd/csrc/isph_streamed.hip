@@ -22,12 +22,12 @@
 // still hold.  A persistent grid that only reads the 210 MB of a 1M-row matrix
 // back and forth does so at 8.2 TB/s, 26 us a pass (6.9 TB/s always forwards).
 //
-// Measured per iteration, launched kernels and here, FP64: 55 and 38 us at 365k
-// rows, 78 and 54 us at 647k, 108 and 84 us at 1.06M; FP32 values with FP64
-// vectors: 50 and 29, 67 and 41, 96 and 61 us.  Of the 84 us the two products
-// take 58 (7.9 TB/s counting the ragged ends of the rows), the exchanges 15.
-// Below 261k rows the resident form is faster (13.7 against 19.8 us at 93k,
-// 20 against 28 us at 255k).
+// Measured per iteration of the solve, launched kernels and here, FP64: 50 and
+// 37 us at 365k rows, 75 and 54 us at 647k, 116 and 83 us at 1.06M; FP32 values
+// with FP64 vectors: 46 and 29, 64 and 40, 87 and 59 us.  Of the 83 us the two
+// products take 58 (7.9 TB/s counting the ragged ends of the rows), the
+// exchanges 15.  Below 261k rows the resident form is faster (9.8 against 19.8
+// us at 93k, 19 against 28 us at 255k).
 //
 // Exchange in two hops: each block publishes its 256-row partials; sixteen
 // waves (one in each of the first sixteen blocks) sum 64 of k_finish's threads
